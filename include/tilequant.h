@@ -84,6 +84,14 @@ int tq_act_quant_fused(const void* x, int64_t x_stride_n, int64_t x_stride_k, in
 int tq_act_quant_token_blocked(const void* x, int64_t x_stride_n, int x_dtype, int n, int k, int8_t* q,
                                float* sx, void* stream);
 
+/* The same for any number of rows n >= 1: one launch up to 512 rows, two above
+ * (workspace = tq_act_absmax_workspace_elems(n, k) floats then).  The operand
+ * format of tq_gemm_mixed_blocked; same scales and code values as
+ * tq_act_quant_fused.  No reference counterpart (row-major codes there,
+ * quant_utils.py:119-134). */
+int tq_act_quant_blocked(const void* x, int64_t x_stride_n, int x_dtype, int n, int k, int8_t* q, float* sx,
+                         float* workspace, int64_t workspace_elems, void* stream);
+
 /* Elements of fp32 workspace tq_act_absmax_scales needs for (n, k); 0 when
  * the scales are produced in a single pass. */
 int64_t tq_act_absmax_workspace_elems(int n, int k);
@@ -195,6 +203,25 @@ int tq_gemm_mixed_rows_planned(const int8_t* x_int8, int64_t x_int8_stride_n, co
 int tq_gemm_prefill_plan(const int32_t* int8_row_ptr, const int32_t* int8_tile_ids,
                          const int32_t* fp16_row_ptr, int n_tr, int n_tc, int32_t* units, int max_units,
                          int* n_first);
+
+/* The GEMM for prompt sizes on token-blocked codes of any number of rows
+ * (tq_act_quant_blocked): x_blocked, 16 ceil(n / 16) * k bytes.  k = 64 * n_tc,
+ * n_tc <= 304, 16-byte aligned x_fp rows (x_fp_stride_n % 8 == 0).  The outputs
+ * are bitwise those of tq_gemm_mixed_rows on the same codes row-major for
+ * n > 64.  row_order (nullable, device, n_slots entries): the row tiles 0 ..
+ * n_tr - 1, each once, and -1 for empty slots; consecutive groups of four
+ * slots share a workgroup, so row tiles with alike 16-bit tile counts are best
+ * neighbours (any such list gives the same outputs).  products / row0 /
+ * rows: TEST-ONLY, as tq_gemm_mixed_rows_products_i32 (NULL otherwise; bf16
+ * only).  Replaces gemm_mixed_rows_splitk (gemm_rows_splitk_64x64.py:225-323)
+ * for MixedLinear inputs of more than 64 rows. */
+int tq_gemm_mixed_blocked(const int8_t* x_blocked, const float* sx, const int8_t* int8_tiles,
+                          const float* int8_scales, const int32_t* int8_tile_ids, const int32_t* int8_row_ptr,
+                          const void* x_fp, int64_t x_fp_stride_n, int x_dtype, const void* fp16_tiles,
+                          const int32_t* fp16_tile_ids, const int32_t* fp16_row_ptr, void* out,
+                          int64_t out_stride_n, int out_dtype, const void* bias, int n, int m, int k, int n_tr,
+                          int n_tc, int tile_layout, const int32_t* row_order, int n_slots, int32_t* products,
+                          int row0, int rows, void* stream);
 
 /* Workspace (fp32 elements, zero-filled before first use, one per stream) that
  * tq_linear_mixed_fused needs for these arguments: the split-K counters and

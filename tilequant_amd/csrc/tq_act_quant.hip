@@ -190,10 +190,11 @@ __global__ void act_scales_finalize_kernel(const float* __restrict__ partial, in
 // round trip.  Vector layout only (unit column stride, 16-byte aligned rows,
 // k a multiple of 64, 8-byte aligned code rows).  Same closed forms as
 // act_scales_finalize_kernel + act_quant_scaled_kernel, bit for bit.
+// nb > 0: codes token-blocked, rows n .. 16 nb - 1 written as zeros.
 template <class T>
 __global__ void __launch_bounds__(kQuantThreads)
 act_quant_block_kernel(XView v, const float* __restrict__ partial, int n_rb, int8_t* __restrict__ q, int64_t ldq,
-                       float* __restrict__ sx) {
+                       float* __restrict__ sx, int nb) {
   __shared__ float scale;
   const int c = blockIdx.x, rb = blockIdx.y, t = threadIdx.x, n_tc = gridDim.x;
   const int row0 = rb * kPartialRows, row1 = min(v.n, row0 + kPartialRows);
@@ -217,7 +218,42 @@ act_quant_block_kernel(XView v, const float* __restrict__ partial, int n_rb, int
 #pragma unroll
   for (int i = 0; i < kPer; ++i) {
     const int row = row0 + t / 8 + i * kRowsPerPass;
-    if (row < row1) *reinterpret_cast<u32x2*>(q + (int64_t)row * ldq + col) = codes8<T>(w[i], cs);
+    if (nb > 0) {
+      if (row < 16 * nb)
+        *reinterpret_cast<u32x2*>(q + blocked_offset(row, col, nb)) = row < row1 ? codes8<T>(w[i], cs) : u32x2{0u, 0u};
+    } else if (row < row1) {
+      *reinterpret_cast<u32x2*>(q + (int64_t)row * ldq + col) = codes8<T>(w[i], cs);
+    }
+  }
+}
+
+// 65 .. 512 rows in one launch: a workgroup of 16 waves per column tile, each
+// thread holding up to four 8-element groups in registers from the absmax to
+// the codes (one pass over the input).  Token-blocked codes, vector layout
+// only.  Same closed form as act_quant_fused_kernel, bit for bit.
+constexpr int kMidThreads = 1024;
+
+template <class T, int G>
+__global__ void __launch_bounds__(kMidThreads)
+act_quant_mid_kernel(XView v, int8_t* __restrict__ q, float* __restrict__ sx, int nb) {
+  __shared__ float red[kMidThreads / kWave];
+  TQ_ARGS_IN_SGPRS("s"(v.x), "s"(v.sn), "s"(v.n), "s"(q), "s"(sx), "s"(nb));
+  constexpr int kRows = kMidThreads / 8;
+  const int c = blockIdx.x, t = threadIdx.x, col = c * kTile + (t % 8) * 8;
+  u32x4 w[G];
+  float m = 0.0f;
+#pragma unroll
+  for (int i = 0; i < G; ++i) w[i] = load8(v, min(t / 8 + i * kRows, v.n - 1), col);
+#pragma unroll
+  for (int i = 0; i < G; ++i) m = max8<T>(w[i], m);   // a clamped row is a row of the tile
+  const float s = act_scale_from_absmax<T>(block_max(m, red, kMidThreads / kWave));
+  const CodeScale cs(s);
+  if (t == 0) sx[c] = s;
+#pragma unroll
+  for (int i = 0; i < G; ++i) {
+    const int row = t / 8 + i * kRows;
+    if (row < 16 * nb)
+      *reinterpret_cast<u32x2*>(q + blocked_offset(row, col, nb)) = row < v.n ? codes8<T>(w[i], cs) : u32x2{0u, 0u};
   }
 }
 
@@ -436,10 +472,48 @@ extern "C" int tq_act_quant_two_level(const void* x, int64_t x_stride_n, int x_d
   const dim3 grid(n_tc, n_rb);
   if (x_dtype == TQ_DTYPE_BF16) {
     hipLaunchKernelGGL(act_absmax_partial_kernel<Bf16>, grid, dim3(kQuantThreads), 0, s, v, workspace, kPartialRows, 0);
-    hipLaunchKernelGGL(act_quant_block_kernel<Bf16>, grid, dim3(kQuantThreads), 0, s, v, workspace, n_rb, q, q_stride_n, sx);
+    hipLaunchKernelGGL(act_quant_block_kernel<Bf16>, grid, dim3(kQuantThreads), 0, s, v, workspace, n_rb, q, q_stride_n, sx, 0);
   } else {
     hipLaunchKernelGGL(act_absmax_partial_kernel<Fp16>, grid, dim3(kQuantThreads), 0, s, v, workspace, kPartialRows, 0);
-    hipLaunchKernelGGL(act_quant_block_kernel<Fp16>, grid, dim3(kQuantThreads), 0, s, v, workspace, n_rb, q, q_stride_n, sx);
+    hipLaunchKernelGGL(act_quant_block_kernel<Fp16>, grid, dim3(kQuantThreads), 0, s, v, workspace, n_rb, q, q_stride_n, sx, 0);
+  }
+  return (int)hipGetLastError();
+}
+
+template <class T>
+static void launch_mid(const XView& v, int8_t* q, float* sx, int nb, hipStream_t s) {
+  const dim3 grid(n_tiles_of(v.k)), block(kMidThreads);
+  if (v.n <= 128) hipLaunchKernelGGL((act_quant_mid_kernel<T, 1>), grid, block, 0, s, v, q, sx, nb);
+  else if (v.n <= 256) hipLaunchKernelGGL((act_quant_mid_kernel<T, 2>), grid, block, 0, s, v, q, sx, nb);
+  else hipLaunchKernelGGL((act_quant_mid_kernel<T, 4>), grid, block, 0, s, v, q, sx, nb);
+}
+
+extern "C" int tq_act_quant_blocked(const void* x, int64_t x_stride_n, int x_dtype, int n, int k, int8_t* q, float* sx,
+                                    float* workspace, int64_t workspace_elems, void* stream) {
+  int rc = check_x(x, x_stride_n, 1, x_dtype, n, k);
+  if (rc) return rc;
+  if (n < 1 || k < kTile || (k % kTile) != 0 || q == nullptr || sx == nullptr) return TQ_ERR_ARG;
+  if ((x_stride_n % 8) != 0 || !aligned16(x) || ((uintptr_t)q & 7u) != 0) return TQ_ERR_ALIGN;
+  if (n <= 64) return tq_act_quant_token_blocked(x, x_stride_n, x_dtype, n, k, q, sx, stream);
+  XView v{static_cast<const uint16_t*>(x), x_stride_n, 1, n, k};
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  const int nb = (n + 15) / 16;
+  const bool bf = x_dtype == TQ_DTYPE_BF16;
+  const int64_t need = tq_act_absmax_workspace_elems(n, k);
+  if (need == 0) {
+    if (bf) launch_mid<Bf16>(v, q, sx, nb, s);
+    else launch_mid<Fp16>(v, q, sx, nb, s);
+    return (int)hipGetLastError();
+  }
+  if (workspace == nullptr || workspace_elems < need) return TQ_ERR_WORKSPACE;
+  const int n_rb = (n + kPartialRows - 1) / kPartialRows;
+  const dim3 grid(n_tiles_of(k), n_rb), block(kQuantThreads);
+  if (bf) {
+    hipLaunchKernelGGL(act_absmax_partial_kernel<Bf16>, grid, block, 0, s, v, workspace, kPartialRows, 0);
+    hipLaunchKernelGGL(act_quant_block_kernel<Bf16>, grid, block, 0, s, v, workspace, n_rb, q, (int64_t)0, sx, nb);
+  } else {
+    hipLaunchKernelGGL(act_absmax_partial_kernel<Fp16>, grid, block, 0, s, v, workspace, kPartialRows, 0);
+    hipLaunchKernelGGL(act_quant_block_kernel<Fp16>, grid, block, 0, s, v, workspace, n_rb, q, (int64_t)0, sx, nb);
   }
   return (int)hipGetLastError();
 }

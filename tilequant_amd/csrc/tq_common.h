@@ -9,6 +9,9 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <atomic>
+#include <type_traits>
+
 #include "../../include/tilequant.h"
 
 namespace tq {
@@ -293,6 +296,42 @@ inline int l2_warm_args(const tq_l2_warm* in, int first, L2Warm& out) {
 __device__ inline void lds_barrier() {
   __builtin_amdgcn_s_waitcnt(0xC07F);
   asm volatile("s_barrier" ::: "memory");
+}
+
+// LDS byte address of a __shared__ object
+__device__ inline uint32_t lds_addr(const void* p) {
+  return static_cast<uint32_t>(reinterpret_cast<uintptr_t>((const __attribute__((address_space(3))) char*)p));
+}
+
+template <int V>
+__device__ inline void wait_vmcnt() {
+  // s_waitcnt with vmcnt = V (gfx9 split field) and expcnt / lgkmcnt at their maxima
+  __builtin_amdgcn_s_waitcnt((V & 0xF) | ((V >> 4) << 14) | (0x7 << 4) | (0xF << 8));
+}
+
+// Column tile of a tile id owned by row tile r (id = r * n_tc + c).  Clamped so
+// that a malformed pack can never index sx / x out of range.
+__device__ inline int col_of(int id, int rbase, int n_tc) {
+  return (int)min((unsigned)(id - rbase), (unsigned)(n_tc - 1));
+}
+
+// LDS DMA of 16 bytes per lane: lane l's bytes land at dst + 16 l (dst wave-uniform).
+__device__ inline void dma16(const void* src, void* dst) { __builtin_amdgcn_global_load_lds(src, dst, 16, 0, 0); }
+
+template <class T> struct TypeTag { using type = T; };
+
+// Dynamic LDS beyond the default per-kernel limit needs that limit raised
+// (gfx950: 160 KiB per workgroup, static + dynamic).  Raised per kernel (the
+// kernel is the template argument) to the largest dynamic size requested so
+// far; a failure is returned so that the launch is not attempted.
+template <auto Kern>
+static hipError_t allow_lds(size_t dyn_bytes) {
+  static std::atomic<size_t> raised{0};
+  if (dyn_bytes <= 32 * 1024 || dyn_bytes <= raised.load(std::memory_order_relaxed)) return hipSuccess;
+  const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(Kern),
+                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)dyn_bytes);
+  if (e == hipSuccess) raised.store(dyn_bytes, std::memory_order_relaxed);
+  return e;
 }
 
 }  // namespace tq

@@ -150,12 +150,6 @@ __device__ inline v4i load_xf(const GemmArgs& a, int row, int col) {
   return v4i{(int)w[0], (int)w[1], (int)w[2], (int)w[3]};
 }
 
-// Column tile of a tile id owned by row tile r (id = r * n_tc + c).  Clamped so
-// that a malformed pack can never index sx / x out of range.
-__device__ inline int col_of(int id, int rbase, int n_tc) {
-  return (int)min((unsigned)(id - rbase), (unsigned)(n_tc - 1));
-}
-
 // Test instantiations (DUMP = true) of the production kernels: the exact
 // INT32 result d of an INT8 tile's v_mfma_i32_16x16x64_i8, before its scale
 // FMA, is also written to a.dump[p][row - dump_r0][col] for the token rows
@@ -1347,21 +1341,10 @@ constexpr int kPfStage = 4096 + kPfXBytes;
 constexpr int kPfStages = 3;
 constexpr int kPfMeta = 512;
 
-// LDS byte address of a __shared__ object
-__device__ inline uint32_t lds_addr(const void* p) {
-  return static_cast<uint32_t>(reinterpret_cast<uintptr_t>((const __attribute__((address_space(3))) char*)p));
-}
-
 __device__ inline int lds_read_i32(uint32_t addr) {
   int v;
   asm volatile("ds_read_b32 %0, %1\n\ts_waitcnt lgkmcnt(0)" : "=&v"(v) : "v"(addr) : "memory");
   return v;
-}
-
-template <int V>
-__device__ inline void wait_vmcnt() {
-  // s_waitcnt with vmcnt = V (gfx9 split field) and expcnt / lgkmcnt at their maxima
-  __builtin_amdgcn_s_waitcnt((V & 0xF) | ((V >> 4) << 14) | (0x7 << 4) | (0xF << 8));
 }
 
 template <class XT, int P, bool DUMP = false>
@@ -1776,7 +1759,6 @@ gemm_prefill_v3_kernel(GemmArgs a) {
 // carrying many 16-bit tiles first so that they do not finish last.  A unit's
 // per-output arithmetic is the same either way.
 constexpr int kP5Threads = 256;
-template <class T> struct TypeTag { using type = T; };
 constexpr int kP5Stages = 3;
 constexpr int kP5MaxCols = 304;   // k <= 19456 (Qwen2.5-7B down: 296 column tiles); LDS 81 KB
 constexpr int kP5OutRow = 272;    // LDS bytes per staged output row (256 + 16: no bank conflicts)
@@ -2290,20 +2272,6 @@ static SplitPlan plan_split(int n, int n_tr, int n_tc, int split_k) {
 static int64_t split_workspace_elems(const SplitPlan& p, int n, int n_tr) {
   const int64_t units = (int64_t)n_tr * (4 / p.jbw);
   return p.S > 1 ? counter_elems((int)units) + units * p.S * n * 64 : 0;
-}
-
-// Dynamic LDS beyond the default per-kernel limit needs that limit raised
-// (gfx950: 160 KiB per workgroup, static + dynamic).  Raised per kernel (the
-// kernel is the template argument) to the largest dynamic size requested so
-// far; a failure is returned so that the launch is not attempted.
-template <auto Kern>
-static hipError_t allow_lds(size_t dyn_bytes) {
-  static std::atomic<size_t> raised{0};
-  if (dyn_bytes <= 32 * 1024 || dyn_bytes <= raised.load(std::memory_order_relaxed)) return hipSuccess;
-  const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(Kern),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)dyn_bytes);
-  if (e == hipSuccess) raised.store(dyn_bytes, std::memory_order_relaxed);
-  return e;
 }
 
 template <auto Kern>

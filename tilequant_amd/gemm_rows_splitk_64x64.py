@@ -86,10 +86,23 @@ class PrefillPlan:
     ``prefill_plan`` builds one from the row pointers; the outputs do not
     depend on it, as long as it covers the weight's row tiles."""
 
-    __slots__ = ("units", "n_first", "n_tr")
+    __slots__ = ("units", "n_first", "n_tr", "row_order")
 
-    def __init__(self, units: torch.Tensor, n_first: int, n_tr: int):
+    def __init__(self, units: torch.Tensor, n_first: int, n_tr: int, row_order: Optional[torch.Tensor] = None):
         self.units, self.n_first, self.n_tr = units, int(n_first), int(n_tr)
+        self.row_order = row_order   # slots of the blocked GEMM (_row_order; None: row tiles in order)
+
+
+def _row_order(rp16: torch.Tensor, n_tr: int, n_tc: int) -> torch.Tensor:
+    """Slots of the blocked GEMM: row tiles by descending 16-bit tile count.
+    Four neighbours share a workgroup and finish together when their counts
+    are alike; those mostly in 16 bits (two thirds of the tiles) are padded with
+    empty slots (-1) to whole workgroups, since beside an INT8 row tile each
+    would wait for the other's phase."""
+    counts = rp16[1:n_tr + 1] - rp16[:n_tr]
+    order = torch.argsort(counts, descending=True, stable=True).to(torch.int32)
+    heavy = int((3 * counts >= 2 * n_tc).sum())
+    return torch.cat((order[:heavy], torch.full((-heavy % 4,), -1, dtype=torch.int32), order[heavy:])).contiguous()
 
 
 def prefill_plan(*, int8_tile_ids: torch.Tensor, int8_row_ptr: torch.Tensor, fp16_row_ptr: torch.Tensor,
@@ -117,7 +130,8 @@ def prefill_plan(*, int8_tile_ids: torch.Tensor, int8_row_ptr: torch.Tensor, fp1
     if rc == 0:
         return None
     dev = device if device is not None else int8_row_ptr.device
-    return PrefillPlan(units[:rc].to(dev), n_first.value, n_tr)
+    order = _row_order(rp16, n_tr, n_tc).to(dev) if rp16 is not None else None
+    return PrefillPlan(units[:rc].to(dev), n_first.value, n_tr, order)
 
 
 def _check_tiles(name: str, t: torch.Tensor, dtype) -> None:
@@ -303,6 +317,88 @@ def linear_mixed_fused(
     else:
         rc = nat.lib().tq_linear_mixed_fused(*args, nat.stream_handle(x_fp.device))
         nat.check(rc, "tq_linear_mixed_fused")
+    return out
+
+
+# Column tiles the blocked GEMM takes (its per-wave column map): k <= 19456.
+BLOCKED_MAX_COLUMN_TILES = 304
+
+
+def gemm_mixed_rows_blocked(
+    *,
+    x_fp: torch.Tensor,
+    x_blocked: torch.Tensor,
+    sx: torch.Tensor,
+    int8_tiles: torch.Tensor,
+    int8_scales: torch.Tensor,
+    int8_tile_ids: torch.Tensor,
+    int8_row_ptr: torch.Tensor,
+    fp16_tiles: torch.Tensor,
+    fp16_tile_ids: torch.Tensor,
+    fp16_row_ptr: torch.Tensor,
+    M: int,
+    K: int,
+    n_tr: int,
+    n_tc: int,
+    out_dtype: torch.dtype,
+    bias: Optional[torch.Tensor] = None,
+    out: Optional[torch.Tensor] = None,
+    tile_layout: str = "row_major",
+    row_order: Optional[torch.Tensor] = None,
+    _products=None,
+) -> torch.Tensor:
+    """``gemm_mixed_rows_splitk`` on the token-blocked codes of
+    ``quantize_activation_blocked``, for prompt sizes (more than 64 rows;
+    ``K == 64 * n_tc``, at most ``BLOCKED_MAX_COLUMN_TILES`` column tiles,
+    16-byte aligned ``x_fp`` rows).  ``row_order`` (optional int32 tensor of
+    the row tiles, each once, and -1 for empty slots) groups the workgroups and
+    does not change the result.
+    ``_products`` is the test-only (int32 [T8, rows, 64], row0, rows) dump."""
+    nat.require_device(x_fp, x_blocked, sx, int8_tiles, int8_scales, int8_tile_ids, int8_row_ptr, fp16_tiles,
+                       fp16_tile_ids, fp16_row_ptr, bias, out, row_order)
+    n = int(x_fp.shape[0])
+    M, K, n_tr, n_tc = int(M), int(K), int(n_tr), int(n_tc)
+    if n <= 64 or K != 64 * n_tc or not 1 <= n_tc <= BLOCKED_MAX_COLUMN_TILES:
+        raise ValueError(f"the blocked GEMM takes more than 64 rows and K = 64 * n_tc <= "
+                         f"{64 * BLOCKED_MAX_COLUMN_TILES}, got {n} rows, K={K}, n_tc={n_tc}")
+    if out is None:
+        out = torch.empty((n, M), device=x_fp.device, dtype=out_dtype)
+    elif tuple(out.shape) != (n, M) or out.dtype != out_dtype or out.stride(1) != 1:
+        raise ValueError("out must be an (N, M) tensor of out_dtype with unit column stride")
+    if (x_blocked.dtype != torch.int8 or x_blocked.dim() != 1 or x_blocked.numel() != 16 * ((n + 15) // 16) * K
+            or not x_blocked.is_contiguous()):
+        raise ValueError("x_blocked must be a flat contiguous int8 tensor of 16 * ceil(N / 16) * K codes")
+    if x_fp.dim() != 2 or x_fp.shape[1] < K or x_fp.stride(1) != 1:
+        raise ValueError("x_fp must be an (N, >=K) tensor with unit column stride")
+    if sx.dtype != torch.float32 or sx.numel() < n_tc or not sx.is_contiguous():
+        raise ValueError("sx must be a contiguous float32 tensor of n_tc scales")
+    _check_tiles("int8_tiles", int8_tiles, torch.int8)
+    has16 = fp16_tiles.numel() != 0
+    if has16:
+        _check_tiles("fp16_tiles", fp16_tiles, x_fp.dtype)
+    if bias is not None and (bias.dtype != out_dtype or not bias.is_contiguous() or bias.numel() < M):
+        raise ValueError("bias must be a contiguous tensor of out_dtype with M entries")
+    if tile_layout not in nat.TQ_LAYOUT:
+        raise ValueError(f"tile_layout must be one of {tuple(nat.TQ_LAYOUT)}, got {tile_layout!r}")
+    for name, t in (("int8_tile_ids", int8_tile_ids), ("int8_row_ptr", int8_row_ptr),
+                    ("fp16_tile_ids", fp16_tile_ids), ("fp16_row_ptr", fp16_row_ptr)):
+        if t.dtype != torch.int32 or not t.is_contiguous():
+            raise ValueError(f"{name} must be a contiguous int32 tensor")
+    if row_order is not None and (row_order.dtype != torch.int32 or not row_order.is_contiguous()
+                                  or row_order.numel() < n_tr or row_order.device != x_fp.device):
+        raise ValueError("row_order must be a contiguous int32 list of the row tiles on the input's device")
+    if M == 0:
+        return out
+    prod, row0, rows = _products if _products is not None else (None, 0, 0)
+    rc = nat.lib().tq_gemm_mixed_blocked(
+        nat.ptr(x_blocked), nat.ptr(sx), nat.ptr(int8_tiles), nat.ptr(int8_scales), nat.ptr(int8_tile_ids),
+        nat.ptr(int8_row_ptr), nat.ptr(x_fp), x_fp.stride(0), nat.dtype_code(x_fp.dtype),
+        nat.ptr(fp16_tiles) if has16 else None, nat.ptr(fp16_tile_ids) if has16 else None,
+        nat.ptr(fp16_row_ptr) if has16 else None, nat.ptr(out), out.stride(0), nat.dtype_code(out_dtype),
+        nat.ptr(bias), n, M, K, n_tr, n_tc, nat.TQ_LAYOUT[tile_layout], nat.ptr(row_order),
+        row_order.numel() if row_order is not None else 0, nat.ptr(prod), row0, rows,
+        nat.stream_handle(x_fp.device))
+    nat.check(rc, "tq_gemm_mixed_blocked")
     return out
 
 

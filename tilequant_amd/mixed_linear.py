@@ -41,10 +41,12 @@ import torch.nn as nn
 
 from . import _native as nat
 from ._config import cfg_value
-from .gemm_rows_splitk_64x64 import (PrefillPlan, _fused_workspace, _workspace, fused_max_tokens,
-                                     gemm_mixed_rows_splitk, linear_mixed_fused, prefill_plan)
+from .gemm_rows_splitk_64x64 import (BLOCKED_MAX_COLUMN_TILES, PrefillPlan, _fused_workspace, _workspace,
+                                     fused_max_tokens, gemm_mixed_rows_blocked, gemm_mixed_rows_splitk,
+                                     linear_mixed_fused, prefill_plan)
 from .pack import Pack, concat_packs_along_rows
-from .quantize_activation import quantize_activation_token_blocked, token_blocked_elems
+from .quantize_activation import (quantize_activation_blocked, quantize_activation_token_blocked,
+                                  token_blocked_elems)
 from .quant_utils import (
     activation_tile_absmax_scales,
     quantize_activation_tile_absmax,
@@ -173,7 +175,8 @@ def _blockable(x_work: torch.Tensor) -> bool:
 
 def _quantize(x_work: torch.Tensor, tile_n: int, blocked: bool) -> Tuple[torch.Tensor, torch.Tensor]:
     if blocked:
-        return quantize_activation_token_blocked(x_work)
+        return (quantize_activation_blocked if x_work.shape[0] > PLAN_MIN_ROWS
+                else quantize_activation_token_blocked)(x_work)
     return quantize_activation_tile_absmax(x_work, tile_n=tile_n)
 
 
@@ -325,6 +328,25 @@ class MixedLinear(nn.Module):
             prefill_plan=self._prefill_plan(int(x_fp.shape[0])), x_int8_layout=x_int8_layout,
         )
 
+    def _prompt_blocked(self, n_rows: int, x_work: torch.Tensor) -> bool:
+        """Whether a prompt-size input runs on token-blocked codes
+        (``gemm_mixed_rows_blocked``): full column tiles, aligned rows.  The
+        other inputs (and those taken in row chunks) keep row-major codes."""
+        return (n_rows > PLAN_MIN_ROWS and self.tile_n == 64 and self.K_orig == 64 * self.n_tc
+                and 1 <= self.n_tc <= BLOCKED_MAX_COLUMN_TILES and x_work.is_cuda and _blockable(x_work))
+
+    def _gemm_prompt(self, x_fp: torch.Tensor, x_blocked: torch.Tensor, sx: torch.Tensor) -> torch.Tensor:
+        out_dtype = self._out_dtype()
+        plan = self._prefill_plan(int(x_fp.shape[0]))
+        return gemm_mixed_rows_blocked(
+            x_fp=x_fp, x_blocked=x_blocked, sx=sx,
+            int8_tiles=self.int8_tiles, int8_scales=self.int8_scales, int8_tile_ids=self.int8_tile_ids,
+            int8_row_ptr=self.int8_row_ptr, fp16_tiles=self.fp16_tiles, fp16_tile_ids=self.fp16_tile_ids,
+            fp16_row_ptr=self.fp16_row_ptr, M=self.M_orig, K=self.K_orig, n_tr=self.n_tr, n_tc=self.n_tc,
+            out_dtype=out_dtype, bias=self._out_bias(out_dtype), tile_layout=self.tile_layout,
+            row_order=None if plan is None else plan.row_order,
+        )
+
     def token_blocked_codes(self, n_rows: int) -> bool:
         """Whether this module quantizes ``n_rows``-row inputs into
         token-blocked codes: where the GEMM's schedule runs faster on them
@@ -468,6 +490,9 @@ class MixedLinear(nn.Module):
         chunk = self._activation_row_chunk_size()
         if 0 < n_rows <= min(self._fused_rows_for_cfg(), chunk):
             y = self._fused_decode(x_work)
+        elif n_rows <= chunk and self._prompt_blocked(n_rows, x_work):
+            x_blocked, sx = _quantize_for(self, x, x_work, True)
+            y = self._gemm_prompt(x_work, x_blocked, sx)
         elif n_rows <= chunk:
             blocked = self.token_blocked_codes(n_rows) and _blockable(x_work)
             x_int8, sx = _quantize_for(self, x, x_work, blocked)

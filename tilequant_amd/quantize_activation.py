@@ -77,6 +77,24 @@ def quantize_activation_token_blocked(x_fp: torch.Tensor) -> Tuple[torch.Tensor,
     return x_q, sx
 
 
+def quantize_activation_blocked(x_fp: torch.Tensor) -> Tuple[torch.Tensor, torch.Tensor]:
+    """``quantize_activation_token_blocked`` for any number of rows (at least
+    one): the operand format of the prompt-size GEMM
+    (``gemm_mixed_rows_blocked``).  One launch up to 512 rows, two above; same
+    scales and code values as ``quantize_activation_tile_absmax``."""
+    _check_x(x_fp)
+    n, k = (int(v) for v in x_fp.shape)
+    if n < 1 or k == 0 or k % 64:
+        raise ValueError(f"token-blocked codes take at least one row and a multiple of 64 columns, got {(n, k)}")
+    x_q = torch.empty((token_blocked_elems(n, k),), device=x_fp.device, dtype=torch.int8)
+    sx = torch.empty((k // 64,), device=x_fp.device, dtype=torch.float32)
+    ws = _absmax_workspace(x_fp, n, k)
+    rc = nat.lib().tq_act_quant_blocked(nat.ptr(x_fp), x_fp.stride(0), nat.dtype_code(x_fp.dtype), n, k, nat.ptr(x_q),
+                                        nat.ptr(sx), nat.ptr(ws), ws.numel(), nat.stream_handle(x_fp.device))
+    nat.check(rc, "tq_act_quant_blocked")
+    return x_q, sx
+
+
 def activation_tile_absmax_scales_64_fused(x_fp: torch.Tensor) -> torch.Tensor:
     """Scales only, over all rows (reference :158-176)."""
     _check_x(x_fp)
