@@ -1,7 +1,9 @@
 """Prompt sizes on token-blocked codes (tq_act_quant_blocked, tq_gemm_mixed_blocked).
 
 The whole-list kernel forms the row-major prefill kernels' sums: bitwise equal
-outputs, and INT32 tile products equal to the oracle's bit for bit.
+outputs.  The split kernel adds W wave partials: outputs within the oracle's
+tolerance (2 bf16 ulp + the fp32 accumulation bound, oracle.numerics), and its
+INT32 tile products equal to the oracle's bit for bit.
 """
 from __future__ import annotations
 
@@ -11,7 +13,7 @@ import numpy as np
 import pytest
 import torch
 
-from helpers import complement, make_w, make_x, oracle_pack, uniform_fp16_ids, values
+from helpers import assert_gemm_close, complement, make_w, make_x, oracle_pack, uniform_fp16_ids, values
 from oracle import native as onat
 from oracle import numerics as nm
 from tilequant_amd.gemm_rows_splitk_64x64 import gemm_mixed_rows_blocked, gemm_mixed_rows_splitk, prefill_plan
@@ -22,6 +24,7 @@ from tilequant_amd.quantize_activation import quantize_activation_blocked
 
 pytestmark = pytest.mark.gpu
 CFG = SimpleNamespace(quant_style="gi", dtype_out="bf16")
+SPLIT_TOKENS, SPLIT_LONG_TOKENS, SPLIT_LONG_TILES = 384, 1280, 96   # the schedule's limits (tq_prefill.hip)
 
 
 def _pack(m, k, ids16, seed, dtype=torch.bfloat16, layout="mfma"):
@@ -72,7 +75,7 @@ def test_blocked_quantizer_matches_the_oracle(n, dtype):
     (513, 704, 4160, 0.3, torch.bfloat16, "mfma", True),       # 65 column tiles: two windows, an odd count
     (1000, 8192, 320, 0.1, torch.bfloat16, "row_major", True),
     (2049, 16384, 128, 0.1, torch.float16, "mfma", False),     # 128-token workgroups
-    (1281, 192, 8192, 0.1, torch.bfloat16, "mfma", False),     # long lists
+    (1281, 192, 8192, 0.1, torch.bfloat16, "mfma", False),     # long lists past the split limit
     (1300, 128, 19456, 0.05, torch.bfloat16, "mfma", False),   # the most column tiles it takes
 ])
 def test_whole_list_kernel_is_bitwise_the_row_major_kernel(n, m, k, frac, dtype, layout, heavy):
@@ -97,6 +100,38 @@ def test_whole_list_kernel_is_bitwise_the_row_major_kernel(n, m, k, frac, dtype,
         assert torch.equal(wide[:, :m], ref) and torch.all(wide[:, m:] == 5)
         y = gemm_mixed_rows_blocked(x_fp=x, x_blocked=xb, sx=sb, row_order=order, **kw)
         assert torch.equal(y, ref)
+
+
+@pytest.mark.parametrize("n,m,k,frac,layout", [
+    (65, 64, 64, 0.0, "mfma"), (65, 200, 640, 0.3, "row_major"), (128, 512, 3072, 0.05, "mfma"),
+    (384, 320, 320, 0.5, "mfma"), (100, 256, 19456, 0.1, "mfma"), (257, 192, 8192, 0.2, "mfma"),
+    (1280, 64, 6144, 0.1, "mfma"), (300, 128, 512, 1.0, "mfma")])
+def test_split_kernel_products_and_outputs(n, m, k, frac, layout):
+    assert n <= (SPLIT_LONG_TOKENS if k // 64 >= SPLIT_LONG_TILES else SPLIT_TOKENS)
+    ids16 = _ids(m, k, frac, seed=n)
+    W, p = _pack(m, k, ids16, seed=m + k, layout=layout)
+    op = oracle_pack(W, ids16)
+    x = make_x(n, k, seed=n + 2)
+    xd = x.cuda()
+    xb, sx = quantize_activation_blocked(xd)
+    q_ref, s_ref = nm.act_quant(values(x))
+    bias = (torch.randn(m, generator=torch.Generator().manual_seed(n)) * 0.5).to(torch.bfloat16)
+    kw = dict(x_fp=xd, x_blocked=xb, sx=sx, **_kw(p, torch.bfloat16, bias.cuda()))
+    y = gemm_mixed_rows_blocked(**kw)
+    assert torch.equal(gemm_mixed_rows_blocked(**kw), y)
+    T8 = int(p.int8_tiles.shape[0])
+    rows = np.unique(np.r_[0:4, n // 2, n - 4:n])
+    if T8:
+        prod = torch.full((T8, n, 64), -2**31, dtype=torch.int32, device="cuda")
+        assert torch.equal(gemm_mixed_rows_blocked(**kw, _products=(prod, 0, n)), y)
+        ref = onat.tile_products_i32(q_ref[rows], op.int8_tiles, op.int8_tile_ids, p.n_tc, K=k)
+        assert np.array_equal(prod[:, torch.from_numpy(rows).cuda()].cpu().numpy(), ref)
+        assert int((prod == -2**31).sum()) == 0
+    w16 = nm.bf16_bits_to_f32(op.fp16_tiles)
+    _, acc, sab = onat.gemm_mixed(q_ref[rows], s_ref, values(x[rows]), op.int8_tiles, op.int8_scales, op.int8_tile_ids,
+                                  op.int8_row_ptr, w16, op.fp16_tile_ids, op.fp16_row_ptr, p.n_tr, p.n_tc, m, k,
+                                  want_f64=True)
+    assert_gemm_close(y[torch.from_numpy(rows).cuda()], acc, sab, p.n_tc, bias=values(bias))
 
 
 @pytest.mark.parametrize("n,m,k", [(600, 320, 640), (2100, 16384, 128)])

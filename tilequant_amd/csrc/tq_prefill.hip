@@ -551,11 +551,281 @@ gemm_prefill_blocked_kernel(PrefillArgs a) {
   else prefill_blocked_body<XT, TB, false, DUMP>(a, lds, mine, n0, any8, lane, wave);
 }
 
+// ---- few tokens: the row tile's list split over the waves of a workgroup ------
+//
+// Workgroup = one row tile x 64 tokens (2 x 2 accumulator blocks per wave).  Its
+// W waves take the tile list round-robin (INT8 positions first, the 16-bit
+// ones continuing the rotation, as the decode kernels do), each fetching its
+// weight tiles and activation operands straight into registers, D tiles
+// ahead, so no wave waits for another until the partial sums are added, in
+// wave order, through LDS.  Bound by the dependent loads before the first tile
+// (range, ids, operands) and, on large grids, by the 8 KiB of operands per tile
+// from L2.  Per Llama-3.2-3B layer at 128 tokens (keep05, four projections):
+// 175 us with four row tiles per workgroup -> 69 us.
+constexpr int kPdRegion = 8192;   // LDS per wave: 64 tokens x 64 16-bit columns, or 32 x 64 fp32 partials
+
+template <class XT, int D, bool DUMP = false>
+__global__ void __launch_bounds__(512)
+    __attribute__((amdgpu_waves_per_eu(DUMP ? 1 : 2, 2)))
+gemm_prefill_split_kernel(PrefillArgs a) {
+  extern __shared__ __align__(16) int8_t lds[];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int W = blockDim.x >> 6;
+  const int n_tc = a.n_tc;
+  // the token blocks of a row tile are dealt to one XCD back to back (workgroup
+  // b runs on XCD b % 8), so its weights cross the fabric once
+  const int ntb = (a.n + 63) / 64;
+  const int group = blockIdx.x >> 3;
+  const int r = (group / ntb) * 8 + (blockIdx.x & 7), n0 = (group % ntb) * 64;
+  if (r >= a.n_tr) return;
+  const int lo8r = a.rp8[r], n8r = a.rp8[r + 1] - lo8r;
+  const int cnt8 = n8r > wave ? (n8r - wave + W - 1) / W : 0;   // this wave's INT8 tiles
+
+  v16f acc[2][2];
+#pragma unroll
+  for (int f = 0; f < 2; ++f)
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) acc[f][t][v] = 0.f;
+
+  const int rowpart = ((lane >> 4) & 1), kpart = lane >> 5, j = lane & 15;
+  if (cnt8 > 0) {
+    int woff[2];
+#pragma unroll
+    for (int f = 0; f < 2; ++f)
+      woff[f] = a.layout == TQ_LAYOUT_MFMA ? (2 * f + rowpart) * 1024 + kpart * 256 + j * 16
+                                           : (f * 32 + (lane & 31)) * 64 + kpart * 16;
+    const int wh = a.layout == TQ_LAYOUT_MFMA ? 512 : 32;
+    const int first_p = lo8r + wave;
+    int xoff[2];                           // token block t's operand, K half 0 (blocks past the last re-read it)
+#pragma unroll
+    for (int t = 0; t < 2; ++t) xoff[t] = min(n0 / 16 + 2 * t + rowpart, a.nb - 1) * 1024 + kpart * 256 + j * 16;
+    const int64_t xcol = (int64_t)a.nb * 1024;
+    v4i w[D][2][2], x[D][2][2];
+    auto load_w = [&](v4i (&d)[2][2], int i) {
+      const int8_t* t = a.w8 + (int64_t)(first_p + min(i, cnt8 - 1) * W) * 4096;
+#pragma unroll
+      for (int f = 0; f < 2; ++f)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) d[f][h] = *reinterpret_cast<const v4i*>(t + woff[f] + h * wh);
+    };
+    auto load_x = [&](v4i (&d)[2][2], int c) {
+      const int8_t* b = a.xq + (int64_t)c * xcol;
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) d[t][h] = *reinterpret_cast<const v4i*>(b + xoff[t] + h * 512);
+    };
+    // lane i of a window: the wave's tile w0 + i (the last one past the end)
+    auto window = [&](int w0, int& c, float& sc) {
+      const int p = first_p + min(w0 + lane, cnt8 - 1) * W;
+      c = col_of(a.ids8[p], r * n_tc, n_tc);
+      sc = a.sx[c] * a.sw8[p];
+    };
+    load_w(w[0], 0);                       // needs no column: in flight while the ids arrive
+    __builtin_amdgcn_sched_barrier(0);
+    int wc, wcn;
+    float wsc, wscn;
+    window(0, wc, wsc);
+    window(64, wcn, wscn);
+    __builtin_amdgcn_sched_barrier(0);
+    // (the same order of loads as in the loop, so that its waits count exactly)
+#pragma unroll
+    for (int d = 0; d < D; ++d) {
+      if (d > 0) load_w(w[d], d);
+      __builtin_amdgcn_sched_barrier(0);
+      load_x(x[d], __builtin_amdgcn_readlane(wc, d));
+      __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma clang loop unroll(disable)
+    for (int i0 = 0; i0 < cnt8; i0 += D) {
+#pragma unroll
+      for (int d = 0; d < D; ++d) {
+        const int i = i0 + d, in = i + D;
+        // tile i's operands: the 8 loads of each of the D - 1 tiles after it
+        // may stay in flight (waiting here, outside the branch, keeps the
+        // compiler from waiting for everything)
+        if constexpr (DUMP) wait_vmcnt<0>();
+        else wait_vmcnt<8 * (D - 1)>();
+        if (i < cnt8) {
+          if (i > 0 && (i & 63) == 0) {
+            wc = wcn;
+            wsc = wscn;
+            window(i + 64, wcn, wscn);
+          }
+          const float sc = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(wsc), i & 63));
+          const int p = first_p + i * W;
+          tile_mac<2>(
+              acc, w[d], x[d], sc, [](int) {},
+              [&](int f, int t, const v16i& m) {
+                if constexpr (DUMP) dump_block(a, p, n0 + 32 * t, 32 * f, lane, m);
+              });
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        const int cn = (in & 63) >= (i & 63) ? __builtin_amdgcn_readlane(wc, in & 63)
+                                             : __builtin_amdgcn_readlane(wcn, in & 63);
+        load_w(w[d], in);
+        load_x(x[d], cn);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    wait_vmcnt<0>();
+  }
+
+  int8_t* region = lds + wave * kPdRegion;
+  if (a.w16 != nullptr) {
+    const int lo16r = a.rp16[r], n16r = a.rp16[r + 1] - lo16r;
+    const int f16 = (wave - n8r % W + W) % W;
+    const int cnt16 = n16r > f16 ? (n16r - f16 + W - 1) / W : 0;
+    const int first_q = lo16r + f16;
+    const int xch = ((lane & 7) ^ (lane >> 3)) * 8;
+    auto fetch_x16 = [&](int c) {          // 64 rows of 128 bytes, 16-byte chunk c of row R at slot c ^ (R % 8)
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const int64_t row = min(n0 + 8 * i + (lane >> 3), a.n - 1);
+        dma16(a.xf + row * a.ldx + c * 64 + xch, region + i * 1024);
+      }
+    };
+    int woff[2];
+#pragma unroll
+    for (int f = 0; f < 2; ++f)
+      woff[f] = a.layout == TQ_LAYOUT_MFMA ? (2 * f + rowpart) * 1024 + kpart * 128 + j * 8
+                                           : (f * 32 + (lane & 31)) * 64 + kpart * 8;
+    v4i w[2][4];
+    auto load_w16 = [&](int q) {
+      const uint16_t* t = a.w16 + (int64_t)q * 4096;
+#pragma unroll
+      for (int f = 0; f < 2; ++f)
+#pragma unroll
+        for (int kc = 0; kc < 4; ++kc)
+          w[f][kc] = *reinterpret_cast<const v4i*>(
+              t + woff[f] + (a.layout == TQ_LAYOUT_MFMA ? (kc >> 1) * 512 + (kc & 1) * 256 : kc * 16));
+    };
+    uint32_t xrd[4];
+#pragma unroll
+    for (int kc = 0; kc < 4; ++kc)
+      xrd[kc] = lds_addr(region) + (lane & 31) * 128 + (((2 * kc + kpart) ^ (lane & 7)) * 16);
+    for (int w0 = 0; w0 < cnt16; w0 += 64) {
+      const int cols = col_of(a.ids16[first_q + min(w0 + lane, cnt16 - 1) * W], r * n_tc, n_tc);
+      const int nq = min(64, cnt16 - w0);
+      fetch_x16(__builtin_amdgcn_readlane(cols, 0));
+      load_w16(first_q + w0 * W);
+      for (int i = 0; i < nq; ++i) {
+        const int in = min(i + 1, nq - 1);
+        wait_vmcnt<0>();
+        v4i xv[2][4];
+        asm volatile(
+            "ds_read_b128 %0, %8\n\t"
+            "ds_read_b128 %1, %9\n\t"
+            "ds_read_b128 %2, %10\n\t"
+            "ds_read_b128 %3, %11\n\t"
+            "ds_read_b128 %4, %8 offset:4096\n\t"
+            "ds_read_b128 %5, %9 offset:4096\n\t"
+            "ds_read_b128 %6, %10 offset:4096\n\t"
+            "ds_read_b128 %7, %11 offset:4096\n\t"
+            "s_waitcnt lgkmcnt(0)"
+            : "=&v"(xv[0][0]), "=&v"(xv[0][1]), "=&v"(xv[0][2]), "=&v"(xv[0][3]), "=&v"(xv[1][0]), "=&v"(xv[1][1]),
+              "=&v"(xv[1][2]), "=&v"(xv[1][3])
+            : "v"(xrd[0]), "v"(xrd[1]), "v"(xrd[2]), "v"(xrd[3])
+            : "memory");
+        __builtin_amdgcn_sched_barrier(0);
+        fetch_x16(__builtin_amdgcn_readlane(cols, in));   // the operands are in registers: refill at once
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int kc = 0; kc < 4; ++kc)
+#pragma unroll
+          for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int f = 0; f < 2; ++f) acc[f][t] = mfma32<XT>(w[f][kc], xv[t][kc], acc[f][t]);
+        __builtin_amdgcn_sched_barrier(0);
+        load_w16(first_q + (w0 + in) * W);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      wait_vmcnt<0>();
+    }
+  }
+
+  // ---- outputs ------------------------------------------------------------------
+  auto round4 = [&](const float* y, int feat) {   // four features of one token, rounded (+ bias, rounded again)
+    u32x2 o;
+    auto go = [&](auto out_tag) {
+      using OT = typename decltype(out_tag)::type;
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        uint32_t y2 = OT::pack2(y[2 * e], y[2 * e + 1]);
+        if (a.bias != nullptr) {
+          const int col = r * 64 + feat + 2 * e;
+          const float b0 = OT::to_f32(a.bias[min(col, a.m - 1)]), b1 = OT::to_f32(a.bias[min(col + 1, a.m - 1)]);
+          y2 = OT::pack2(OT::to_f32((uint16_t)y2) + b0, OT::to_f32((uint16_t)(y2 >> 16)) + b1);
+        }
+        o[e] = y2;
+      }
+    };
+    if (a.out_bf16) go(TypeTag<Bf16>{});
+    else go(TypeTag<Fp16>{});
+    return o;
+  };
+  {
+    // Partial sums through LDS, one 32-feature half at a time: chunk
+    // (t, g) of wave w is 64 lanes x 4 features, summed over the waves in
+    // wave order by wave (chunk % W).
+    int8_t* staged = lds + W * kPdRegion;
+#pragma unroll
+    for (int f = 0; f < 2; ++f) {
+      __syncthreads();   // the regions are free (16-bit operands read; the previous half summed)
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+          *reinterpret_cast<v4f*>(region + (t * 4 + g) * 1024 + lane * 16) =
+              v4f{acc[f][t][4 * g], acc[f][t][4 * g + 1], acc[f][t][4 * g + 2], acc[f][t][4 * g + 3]};
+      __syncthreads();
+      for (int q = wave; q < 8; q += W) {
+        v4f s = *reinterpret_cast<const v4f*>(lds + q * 1024 + lane * 16);
+        for (int u = 1; u < W; ++u) {
+          const v4f b = *reinterpret_cast<const v4f*>(lds + u * kPdRegion + q * 1024 + lane * 16);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) s[e] += b[e];
+        }
+        const int t = q >> 2, g = q & 3, row = t * 32 + (lane & 31), feat = f * 32 + 8 * g + 4 * kpart;
+        const float y[4] = {s[0], s[1], s[2], s[3]};
+        *reinterpret_cast<u32x2*>(staged + row * 128 + (((f * 4 + g) ^ (row & 7)) * 16) + kpart * 8) = round4(y, feat);
+      }
+    }
+    __syncthreads();
+    store_rows(a, staged, r, n0, 64, threadIdx.x, blockDim.x);
+  }
+}
+
 }  // namespace tq
 
 using namespace tq;
 
-// 64 or 128 tokens per workgroup (the same sums): the cheaper grid
+// Schedule of n tokens.  Which sums are formed (W waves' partials, or one
+// accumulator per output) depends on n and n_tc only, so stacked projections
+// stay bitwise equal to their members.
+//
+// Split lists while whole-list workgroups leave most of the chip waiting for
+// each wave's serial walk (0.56 us per tile).  Measured on MI355X, us per launch,
+// whole list -> split over 4 waves, 96 / 192 / 384 / 512 tokens:
+//   Llama-3.2-3B Q/K/V   32 -> 14   33 -> 14   33 -> 19   34 -> 27
+//     O                  33 -> 13   33 -> 14   33 -> 18   33 -> 18
+//     Gate/Up            35 -> 20   35 -> 31   47 -> 49   50 -> 63
+//   Qwen2.5-7B Gate/Up   56 -> 55   90 -> 74   96 -> 130  142 -> 179
+// so the layer's three together gain up to about 400 tokens.  Long lists (Down)
+// longer, 192 / 1024 / 1500 tokens: Llama 73 -> 23, 77 -> 54, 103 -> 87;
+// Qwen2.5-7B 160 -> 44, 173 -> 139, 229 -> 219; 14B 120 -> 36, 173 -> 131, 183 ->
+// 221.  Eight waves where the list is long and the grid small (192 tokens: 21,
+// 38 and 32 against 23, 44 and 36 us; at 384 37, 71, 59 against 32, 64, 53).
+constexpr int kSplitTokens = 384, kSplitLongTokens = 1280, kSplitLongTiles = 96, kSplitWideTokens = 256;
+static int split_waves(int n, int n_tc) {
+  if (n > (n_tc >= kSplitLongTiles ? kSplitLongTokens : kSplitTokens)) return 0;
+  return n_tc >= kSplitLongTiles && n <= kSplitWideTokens ? 8 : 4;
+}
+
+// 64 or 128 tokens per workgroup otherwise (the same sums): the cheaper grid
 // by the time of the most loaded CU.  A CU runs three 64-token workgroups or two
 // 128-token ones together; measured on MI355X with 48-tile lists (us), 64
 // tokens: 35 for one workgroup per CU, 51 for two, 68 for three; 128 tokens: 55
@@ -576,6 +846,16 @@ static int blocked_tb(int n, int units) {
 
 template <class XT, bool DUMP>
 static hipError_t launch_blocked(PrefillArgs a, hipStream_t s) {
+  if (const int W = split_waves(a.n, a.n_tc)) {
+    constexpr auto kern = gemm_prefill_split_kernel<XT, 2, DUMP>;
+    const int64_t blocks = 8ll * ((a.n_tr + 7) / 8) * ((a.n + 63) / 64);
+    if (blocks >= (1ll << 31)) return hipErrorInvalidValue;
+    const size_t lds = (size_t)W * kPdRegion + 8192;
+    const hipError_t e = allow_lds<kern>(lds);
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(64 * W), lds, s, a);
+    return hipGetLastError();
+  }
   a.n_units = (a.n_slots + 3) / 4;
   const int tb = blocked_tb(a.n, a.n_units);
   const int64_t blocks = (int64_t)a.n_units * ((a.n + 32 * tb - 1) / (32 * tb));
