@@ -223,6 +223,45 @@ int tq_gemm_mixed_blocked(const int8_t* x_blocked, const float* sx, const int8_t
                           int n_tc, int tile_layout, const int32_t* row_order, int n_slots, int32_t* products,
                           int row0, int rows, void* stream);
 
+/* Host function: slots of tq_gemm_mixed_blocked for one packed weight, from a HOST
+ * copy of its 16-bit row pointers: the row tiles by descending 16-bit tile
+ * count, those with at least two thirds of their n_tc tiles in 16 bits first
+ * and padded with empty slots (-1) to whole groups of four (beside an INT8 row
+ * tile each would wait for the other's phase).  Writes into slots[0 ..
+ * max_slots), max_slots >= n_tr + 3; returns the slot count or TQ_ERR_ARG. */
+int tq_gemm_row_order(const int32_t* fp16_row_ptr, int n_tr, int n_tc, int32_t* slots, int max_slots);
+
+/* One MixedLinear forward at prompt sizes (n > 64): tq_act_quant_blocked into
+ * x_blocked / sx (with quantize = 1; 0: they hold x's codes already, from a
+ * sibling projection) followed by tq_gemm_mixed_blocked -- the same launches,
+ * arguments and results.  The caller validates once and patches the per-call
+ * fields of a copy.  Counterpart of the reference's CachedLauncher
+ * (src/kernels/triton/launch.py:9-79) for prompts. */
+typedef struct tq_prompt_desc {
+  /* per call */
+  const void* x;          /* [n, k] activations, x_dtype, row stride x_stride */
+  void* out;              /* [n, m] out_dtype, row stride out_stride */
+  int8_t* x_blocked;      /* 16 ceil(n / 16) * k codes */
+  float* sx;              /* [n_tc] */
+  float* workspace;       /* tq_act_absmax_workspace_elems(n, k) floats, or NULL when that is 0 */
+  int64_t workspace_elems;
+  void* stream;
+  /* fixed */
+  int64_t x_stride, out_stride;
+  int quantize, n, m, k, n_tr, n_tc, x_dtype, out_dtype, tile_layout, n_slots;
+  const int8_t* int8_tiles;
+  const float* int8_scales;
+  const int32_t* int8_tile_ids;
+  const int32_t* int8_row_ptr;
+  const void* fp16_tiles; /* NULL when the pack has no 16-bit tiles */
+  const int32_t* fp16_tile_ids;
+  const int32_t* fp16_row_ptr;
+  const void* bias;       /* out_dtype [m] or NULL */
+  const int32_t* row_order; /* n_slots entries, or NULL */
+} tq_prompt_desc;
+
+int tq_prompt_forward(const tq_prompt_desc* d);
+
 /* Workspace (fp32 elements, zero-filled before first use, one per stream) that
  * tq_linear_mixed_fused needs for these arguments: the split-K counters and
  * partials (split_k > 1), or the cooperative launch's counters, codes and

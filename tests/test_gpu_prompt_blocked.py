@@ -185,6 +185,37 @@ def test_mixed_linear_prompts_group_capture_and_plan(n):
             assert torch.equal(y, stacked)
 
 
+def test_mixed_linear_prompt_descriptors_follow_their_module():
+    """Cached prompt descriptors: siblings share one quantization under
+    inference mode, in-place bias and input updates are seen, a replaced weight
+    is used, and a module still copies."""
+    import copy
+
+    _, p = _pack(256, 320, _ids(256, 320, 0.1, seed=1), seed=1)
+    x = make_x(700, 320, seed=3).cuda()
+    lin = MixedLinear(p, torch.ones(256, device="cuda", dtype=torch.float16), CFG)   # a bias of another dtype
+    plain = lambda mod, v: gemm_mixed_rows_splitk(   # noqa: E731
+        x_fp=v, x_int8=quantize_activation_tile_absmax(v)[0], sx=quantize_activation_tile_absmax(v)[1],
+        **_kw(mod.to_pack(), torch.bfloat16, mod.bias.to(torch.bfloat16)))
+    twin = copy.deepcopy(lin)
+    with torch.inference_mode():
+        assert torch.equal(lin(x), plain(lin, x)) and torch.equal(twin(x), plain(lin, x))
+        lin.bias.mul_(3)
+        assert torch.equal(lin(x), plain(lin, x))
+    y = x.clone()
+    assert torch.equal(lin(y), plain(lin, y))
+    y.mul_(0.5)
+    assert torch.equal(lin(y), plain(lin, y))
+    assert torch.equal(lin(y.view(7, 100, 320)).view(700, 256), plain(lin, y))
+    other = copy.deepcopy(lin)
+    for name in ("int8_tiles", "int8_scales", "fp16_tiles"):
+        setattr(other, name, getattr(other, name) * 2 if name != "int8_tiles" else getattr(other, name).clone())
+    assert torch.equal(other(y), plain(other, y)) and not torch.equal(other(y), lin(y))
+    wide = torch.zeros((700, 384), device="cuda", dtype=torch.bfloat16)
+    wide[:, :320] = y                                  # not contiguous: copied first, as before
+    assert torch.equal(lin(wide[:, :320]), plain(lin, y))
+
+
 def test_blocked_gemm_refuses_what_it_cannot_take():
     _, p = _pack(128, 128, np.zeros(0, np.int64), seed=1)
     x = make_x(65, 128, seed=2).cuda()

@@ -69,6 +69,7 @@ _SIGNATURES = {
                                         _i, _i, _i, _i, _i,
                                         _i, _i, _p, _i64,
                                         _p, _i, _i, _p]),
+    "tq_gemm_row_order": (_i, [_p, _i, _i, _p, _i]),
     "tq_gemm_prefill_plan": (_i, [_p, _p, _p, _i, _i, _p, _i, ctypes.POINTER(_i)]),
     "tq_linear_mixed_fused": (_i, [_p, _i64, _i,
                                    _p, _p, _p, _p,
@@ -137,6 +138,23 @@ class LinearDesc(ctypes.Structure):
 
 
 _SIGNATURES["tq_linear_forward"] = (_i, [ctypes.POINTER(LinearDesc)])
+
+
+class PromptDesc(ctypes.Structure):
+    """Mirror of tq_prompt_desc (include/tilequant.h)."""
+
+    _fields_ = [
+        ("x", _p), ("out", _p), ("x_blocked", _p), ("sx", _p), ("workspace", _p), ("workspace_elems", _i64),
+        ("stream", _p),
+        ("x_stride", _i64), ("out_stride", _i64),
+        ("quantize", _i), ("n", _i), ("m", _i), ("k", _i), ("n_tr", _i), ("n_tc", _i), ("x_dtype", _i),
+        ("out_dtype", _i), ("tile_layout", _i), ("n_slots", _i),
+        ("int8_tiles", _p), ("int8_scales", _p), ("int8_tile_ids", _p), ("int8_row_ptr", _p),
+        ("fp16_tiles", _p), ("fp16_tile_ids", _p), ("fp16_row_ptr", _p), ("bias", _p), ("row_order", _p),
+    ]
+
+
+_SIGNATURES["tq_prompt_forward"] = (_i, [ctypes.POINTER(PromptDesc)])
 
 
 class L2Warm(ctypes.Structure):

@@ -5,6 +5,9 @@
 // fp32 accumulator per output, the INT8 tiles of a row tile by column (exact
 // INT32 tile product, then one FMA by sx[c] * sw[t]), then its 16-bit tiles by
 // position (the reference's loop, gemm_rows_splitk_64x64.py:125-153).
+#include <algorithm>
+#include <vector>
+
 #include "tq_common.h"
 
 namespace tq {
@@ -904,4 +907,31 @@ extern "C" int tq_gemm_mixed_blocked(const int8_t* x_blocked, const float* sx, c
   else if (x_dtype == TQ_DTYPE_BF16) e = launch_blocked<Bf16, false>(a, s);
   else e = launch_blocked<Fp16, false>(a, s);
   return (int)e;
+}
+
+extern "C" int tq_prompt_forward(const tq_prompt_desc* d) {
+  if (d == nullptr) return TQ_ERR_ARG;
+  if (d->quantize) {
+    const int rc = tq_act_quant_blocked(d->x, d->x_stride, d->x_dtype, d->n, d->k, d->x_blocked, d->sx, d->workspace,
+                                        d->workspace_elems, d->stream);
+    if (rc != 0) return rc;
+  }
+  return tq_gemm_mixed_blocked(d->x_blocked, d->sx, d->int8_tiles, d->int8_scales, d->int8_tile_ids, d->int8_row_ptr,
+                               d->x, d->x_stride, d->x_dtype, d->fp16_tiles, d->fp16_tile_ids, d->fp16_row_ptr, d->out,
+                               d->out_stride, d->out_dtype, d->bias, d->n, d->m, d->k, d->n_tr, d->n_tc,
+                               d->tile_layout, d->row_order, d->n_slots, nullptr, 0, 0, d->stream);
+}
+
+extern "C" int tq_gemm_row_order(const int32_t* fp16_row_ptr, int n_tr, int n_tc, int32_t* slots, int max_slots) {
+  if (fp16_row_ptr == nullptr || slots == nullptr || n_tr < 1 || n_tc < 1 || max_slots < n_tr + 3) return TQ_ERR_ARG;
+  std::vector<int32_t> order((size_t)n_tr);
+  for (int r = 0; r < n_tr; ++r) order[r] = r;
+  auto count = [&](int r) { return fp16_row_ptr[r + 1] - fp16_row_ptr[r]; };
+  std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return count(a) > count(b); });
+  int n = 0;
+  size_t i = 0;
+  for (; i < order.size() && 3 * (int64_t)count(order[i]) >= 2 * (int64_t)n_tc; ++i) slots[n++] = order[i];
+  while (n % 4 != 0) slots[n++] = -1;
+  for (; i < order.size(); ++i) slots[n++] = order[i];
+  return n;
 }

@@ -90,19 +90,7 @@ class PrefillPlan:
 
     def __init__(self, units: torch.Tensor, n_first: int, n_tr: int, row_order: Optional[torch.Tensor] = None):
         self.units, self.n_first, self.n_tr = units, int(n_first), int(n_tr)
-        self.row_order = row_order   # slots of the blocked GEMM (_row_order; None: row tiles in order)
-
-
-def _row_order(rp16: torch.Tensor, n_tr: int, n_tc: int) -> torch.Tensor:
-    """Slots of the blocked GEMM: row tiles by descending 16-bit tile count.
-    Four neighbours share a workgroup and finish together when their counts
-    are alike; those mostly in 16 bits (two thirds of the tiles) are padded with
-    empty slots (-1) to whole workgroups, since beside an INT8 row tile each
-    would wait for the other's phase."""
-    counts = rp16[1:n_tr + 1] - rp16[:n_tr]
-    order = torch.argsort(counts, descending=True, stable=True).to(torch.int32)
-    heavy = int((3 * counts >= 2 * n_tc).sum())
-    return torch.cat((order[:heavy], torch.full((-heavy % 4,), -1, dtype=torch.int32), order[heavy:])).contiguous()
+        self.row_order = row_order   # slots of the blocked GEMM (tq_gemm_row_order; None: row tiles in order)
 
 
 def prefill_plan(*, int8_tile_ids: torch.Tensor, int8_row_ptr: torch.Tensor, fp16_row_ptr: torch.Tensor,
@@ -119,19 +107,23 @@ def prefill_plan(*, int8_tile_ids: torch.Tensor, int8_row_ptr: torch.Tensor, fp1
     rp16 = fp16_row_ptr.detach().to("cpu", torch.int32).contiguous() if fp16_row_ptr.numel() else None
     if rp8.numel() < n_tr + 1 or (rp16 is not None and rp16.numel() < n_tr + 1):
         raise ValueError("row pointers must have n_tr + 1 entries")
-    units = torch.empty(max(n_tr, 1), dtype=torch.int32)
+    units = torch.empty(2 * max(n_tr, 1) + 3, dtype=torch.int32)   # the units, then the blocked GEMM's slots
     n_first = ctypes.c_int(0)
     rc = nat.lib().tq_gemm_prefill_plan(
         rp8.data_ptr(), ids8.data_ptr() if ids8.numel() else None,
-        rp16.data_ptr() if rp16 is not None else None, n_tr, n_tc, units.data_ptr(), units.numel(),
+        rp16.data_ptr() if rp16 is not None else None, n_tr, n_tc, units.data_ptr(), n_tr,
         ctypes.byref(n_first))
     if rc < 0:   # a count otherwise
         nat.check(rc, "tq_gemm_prefill_plan")
     if rc == 0:
         return None
-    dev = device if device is not None else int8_row_ptr.device
-    order = _row_order(rp16, n_tr, n_tc).to(dev) if rp16 is not None else None
-    return PrefillPlan(units[:rc].to(dev), n_first.value, n_tr, order)
+    slots = 0
+    if rp16 is not None:
+        slots = nat.lib().tq_gemm_row_order(rp16.data_ptr(), n_tr, n_tc, units[rc:].data_ptr(), n_tr + 3)
+        if slots < 0:
+            nat.check(slots, "tq_gemm_row_order")
+    both = units[:rc + slots].to(device if device is not None else int8_row_ptr.device)
+    return PrefillPlan(both[:rc], n_first.value, n_tr, both[rc:] if slots else None)
 
 
 def _check_tiles(name: str, t: torch.Tensor, dtype) -> None:
