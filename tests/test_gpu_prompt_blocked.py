@@ -105,7 +105,9 @@ def test_whole_list_kernel_is_bitwise_the_row_major_kernel(n, m, k, frac, dtype,
 @pytest.mark.parametrize("n,m,k,frac,layout", [
     (65, 64, 64, 0.0, "mfma"), (65, 200, 640, 0.3, "row_major"), (128, 512, 3072, 0.05, "mfma"),
     (384, 320, 320, 0.5, "mfma"), (100, 256, 19456, 0.1, "mfma"), (257, 192, 8192, 0.2, "mfma"),
-    (1280, 64, 6144, 0.1, "mfma"), (300, 128, 512, 1.0, "mfma")])
+    (1280, 64, 6144, 0.1, "mfma"), (300, 128, 512, 1.0, "mfma"),
+    # more than 128 row tiles x 64-token blocks: whole row tiles per workgroup
+    (65, 4160, 192, 0.4, "mfma"), (384, 1500, 256, 0.3, "row_major"), (200, 3072, 6144, 0.02, "mfma")])
 def test_split_kernel_products_and_outputs(n, m, k, frac, layout):
     assert n <= (SPLIT_LONG_TOKENS if k // 64 >= SPLIT_LONG_TILES else SPLIT_TOKENS)
     ids16 = _ids(m, k, frac, seed=n)

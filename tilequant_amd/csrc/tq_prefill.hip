@@ -51,7 +51,7 @@ __device__ inline v16f mfma32<Fp16>(v4i av, v4i bv, v16f c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(v8h, av), __builtin_bit_cast(v8h, bv), c, 0, 0, 0);
 }
 
-// One INT8 tile's 64 features x 32 NT tokens: exact INT32 products (two chained
+// One INT8 tile's 32 FB features x 32 NT tokens: exact INT32 products (two chained
 // 32x32x32 MFMAs per 32 x 32 block), then acc = fma((float)d, sc, acc) per
 // element.  The MFMAs of block b + 1 are issued before the conversions of block
 // b, so a wave alone on its SIMD does not sit out the MFMA latency, and each
@@ -59,30 +59,28 @@ __device__ inline v16f mfma32<Fp16>(v4i av, v4i bv, v16f c) {
 // v_fma of another issue together; measured 2.4 cycles per instruction for the
 // alternating stream against 4.3 for either kind alone).  `ready(t)` waits for
 // token block t's operands; `seen(f, t, d)` is the test dump.
-template <int NT, class Ready, class Seen>
-__device__ __attribute__((always_inline)) inline void tile_mac(v16f (&acc)[2][NT], const v4i (&w)[2][2],
+template <int FB, int NT, class Ready, class Seen>
+__device__ __attribute__((always_inline)) inline void tile_mac(v16f (&acc)[FB][NT], const v4i (&w)[FB][2],
                                                                v4i (&x)[NT][2], float sc, Ready&& ready, Seen&& seen) {
   v16i d[2];
-  auto products = [&](int b) {
-    const v16i z = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-    d[b & 1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(w[b & 1][0], x[b >> 1][0], z, 0, 0, 0);
-    d[b & 1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(w[b & 1][1], x[b >> 1][1], d[b & 1], 0, 0, 0);
-  };
 #pragma unroll
-  for (int b = 0; b <= 2 * NT; ++b) {
-    if (b < 2 * NT) {
-      if ((b & 1) == 0) ready(b >> 1);
-      products(b);
+  for (int b = 0; b <= FB * NT; ++b) {
+    if (b < FB * NT) {
+      const int f = b % FB, t = b / FB;
+      if (f == 0) ready(t);
+      const v16i z = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+      d[b & 1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(w[f][0], x[t][0], z, 0, 0, 0);
+      d[b & 1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(w[f][1], x[t][1], d[b & 1], 0, 0, 0);
       __builtin_amdgcn_sched_barrier(0);
     }
     if (b > 0) {
-      const int f = (b - 1) & 1, t = (b - 1) >> 1;
-      seen(f, t, d[f]);
+      const int f = (b - 1) % FB, t = (b - 1) / FB;
+      seen(f, t, d[(b - 1) & 1]);
       float c[16];
 #pragma unroll
       for (int v = 0; v <= 16; ++v) {
         if (v < 16) {
-          c[v] = (float)d[f][v];
+          c[v] = (float)d[(b - 1) & 1][v];
           __builtin_amdgcn_sched_barrier(0);
         }
         if (v > 0) {
@@ -104,12 +102,14 @@ __device__ inline void dump_block(const PrefillArgs& a, int p, int row0, int f0,
 }
 
 // `rows` staged output rows of row tile r (128 bytes each, 16-byte chunk c of
-// row R at slot c ^ (R % 8)) from token n0 on, by `threads` threads.
+// row R at slot c ^ (R % 8)) from token n0 on, by `threads` threads: CHUNKS
+// chunks of each row from chunk ch0 on.
+template <int CHUNKS = 8>
 __device__ inline void store_rows(const PrefillArgs& a, const int8_t* staged, int r, int n0, int rows, int tid,
-                                  int threads) {
+                                  int threads, int ch0 = 0) {
 #pragma unroll 4
-  for (int q = tid; q < rows * 8; q += threads) {
-    const int rr = q >> 3, ch = q & 7, row = n0 + rr, col = r * 64 + ch * 8;
+  for (int q = tid; q < rows * CHUNKS; q += threads) {
+    const int rr = q / CHUNKS, ch = ch0 + q % CHUNKS, row = n0 + rr, col = r * 64 + ch * 8;
     const v4i val = *reinterpret_cast<const v4i*>(staged + rr * 128 + ((ch ^ (rr & 7)) * 16));
     if (row >= a.n || col >= a.m) continue;
     uint16_t* dst = a.out + (int64_t)row * a.ldo + col;
@@ -276,7 +276,7 @@ __device__ __attribute__((always_inline)) inline void prefill_blocked_body(const
               : "memory");
         }
         const int p = DUMP ? pw[s] : 0;
-        tile_mac<TB>(
+        tile_mac<2, TB>(
             acc, ws, x, sc,
             [&](int t) {
               // LDS reads return in order: token block t has landed when at
@@ -556,18 +556,22 @@ gemm_prefill_blocked_kernel(PrefillArgs a) {
 
 // ---- few tokens: the row tile's list split over the waves of a workgroup ------
 //
-// Workgroup = one row tile x 64 tokens (2 x 2 accumulator blocks per wave).  Its
-// W waves take the tile list round-robin (INT8 positions first, the 16-bit
+// Workgroup = one row tile (FB = 2) or half of one (FB = 1) x 64 tokens: FB x 2
+// accumulator blocks per wave.  Its W waves take the tile list round-robin (INT8 positions first, the 16-bit
 // ones continuing the rotation, as the decode kernels do), each fetching its
 // weight tiles and activation operands straight into registers, D tiles
 // ahead, so no wave waits for another until the partial sums are added, in
-// wave order, through LDS.  Bound by the dependent loads before the first tile
-// (range, ids, operands) and, on large grids, by the 8 KiB of operands per tile
-// from L2.  Per Llama-3.2-3B layer at 128 tokens (keep05, four projections):
-// 175 us with four row tiles per workgroup -> 69 us.
-constexpr int kPdRegion = 8192;   // LDS per wave: 64 tokens x 64 16-bit columns, or 32 x 64 fp32 partials
+// wave order, through LDS.  The first 16-bit tile's operands are fetched into the
+// wave's LDS before the INT8 tiles are walked.  Bound by what a CU keeps in
+// flight: cold weights arrive at about 48 GB/s per CU (Llama-3.2-3B Down, 1 MiB of
+// operands per workgroup, takes 25 us on 48 CUs and on 144), so small grids are
+// spread over more CUs by halving the row tiles.  Per Llama-3.2-3B layer at 128
+// tokens (keep05, four projections, cold weights): 185 us with four row tiles per
+// workgroup -> 68 us.
+constexpr int kPdAhead = 2;        // tiles in flight per wave beyond the one multiplied (3 and 4: up to 20% slower)
+constexpr int kPdRegion = 16384;   // LDS per wave: a 16-bit tile and its activation rows, or 64 x 64 fp32 partials
 
-template <class XT, int D, bool DUMP = false>
+template <class XT, int FB, int D, bool DUMP = false>
 __global__ void __launch_bounds__(512)
     __attribute__((amdgpu_waves_per_eu(DUMP ? 1 : 2, 2)))
 gemm_prefill_split_kernel(PrefillArgs a) {
@@ -579,38 +583,72 @@ gemm_prefill_split_kernel(PrefillArgs a) {
   // the token blocks of a row tile are dealt to one XCD back to back (workgroup
   // b runs on XCD b % 8), so its weights cross the fabric once
   const int ntb = (a.n + 63) / 64;
-  const int group = blockIdx.x >> 3;
-  const int r = (group / ntb) * 8 + (blockIdx.x & 7), n0 = (group % ntb) * 64;
+  constexpr int kParts = 2 / FB;           // workgroups sharing a row tile
+  const int group = blockIdx.x >> 3, part = group % (kParts * ntb);
+  const int r = (group / (kParts * ntb)) * 8 + (blockIdx.x & 7), n0 = (part / kParts) * 64, f0 = (part % kParts) * 32;
   if (r >= a.n_tr) return;
   const int lo8r = a.rp8[r], n8r = a.rp8[r + 1] - lo8r;
   const int cnt8 = n8r > wave ? (n8r - wave + W - 1) / W : 0;   // this wave's INT8 tiles
+  const int32_t* rp16 = a.w16 != nullptr ? a.rp16 : a.rp8;
+  const int lo16r = rp16[r], n16r = a.w16 != nullptr ? rp16[r + 1] - lo16r : 0;
+  const int f16 = (wave - n8r % W + W) % W;
+  const int cnt16 = n16r > f16 ? (n16r - f16 + W - 1) / W : 0;  // ... and 16-bit tiles
+  const int first_q = lo16r + f16;
+  int8_t* region = lds + wave * kPdRegion;
+  const int rowpart = ((lane >> 4) & 1), kpart = lane >> 5, j = lane & 15;
 
-  v16f acc[2][2];
+  // 16-bit tile q of column tile c into the wave's region: 64 activation rows of
+  // 128 bytes (16-byte chunk c of row R at slot c ^ (R % 8)), then the tile in
+  // MFMA order (one KiB per 16 features x 32 columns).
+  auto fetch16 = [&](int q, int c) {
+    const int xch = ((lane & 7) ^ (lane >> 3)) * 8;
 #pragma unroll
-  for (int f = 0; f < 2; ++f)
+    for (int i = 0; i < 8; ++i) {
+      const int64_t row = min(n0 + 8 * i + (lane >> 3), a.n - 1);
+      dma16(a.xf + row * a.ldx + c * 64 + xch, region + i * 1024);
+    }
+    const uint16_t* t = a.w16 + (int64_t)q * 4096 + f0 * 64;
+    const int in_row = j * 64 + (lane >> 4) * 8;
+#pragma unroll
+    for (int i = 0; i < 4 * FB; ++i)       // i = 2 jb + h
+      dma16(a.layout == TQ_LAYOUT_MFMA ? t + i * 512 + lane * 8 : t + (i >> 1) * 1024 + (i & 1) * 32 + in_row,
+            region + 8192 + i * 1024);
+  };
+  auto cols16 = [&](int w0) {              // lane i: column of the wave's 16-bit tile w0 + i
+    return col_of(a.ids16[first_q + min(w0 + lane, cnt16 - 1) * W], r * n_tc, n_tc);
+  };
+  // The first one's operands land while the INT8 tiles are multiplied.
+  int wcol16 = 0;
+  if (cnt16 > 0) {
+    wcol16 = cols16(0);
+    fetch16(first_q, __builtin_amdgcn_readlane(wcol16, 0));
+  }
+
+  v16f acc[FB][2];
+#pragma unroll
+  for (int f = 0; f < FB; ++f)
 #pragma unroll
     for (int t = 0; t < 2; ++t)
 #pragma unroll
       for (int v = 0; v < 16; ++v) acc[f][t][v] = 0.f;
 
-  const int rowpart = ((lane >> 4) & 1), kpart = lane >> 5, j = lane & 15;
   if (cnt8 > 0) {
-    int woff[2];
+    int woff[FB];
 #pragma unroll
-    for (int f = 0; f < 2; ++f)
-      woff[f] = a.layout == TQ_LAYOUT_MFMA ? (2 * f + rowpart) * 1024 + kpart * 256 + j * 16
-                                           : (f * 32 + (lane & 31)) * 64 + kpart * 16;
+    for (int f = 0; f < FB; ++f)
+      woff[f] = f0 * 64 + (a.layout == TQ_LAYOUT_MFMA ? (2 * f + rowpart) * 1024 + kpart * 256 + j * 16
+                                                      : (f * 32 + (lane & 31)) * 64 + kpart * 16);
     const int wh = a.layout == TQ_LAYOUT_MFMA ? 512 : 32;
     const int first_p = lo8r + wave;
     int xoff[2];                           // token block t's operand, K half 0 (blocks past the last re-read it)
 #pragma unroll
     for (int t = 0; t < 2; ++t) xoff[t] = min(n0 / 16 + 2 * t + rowpart, a.nb - 1) * 1024 + kpart * 256 + j * 16;
     const int64_t xcol = (int64_t)a.nb * 1024;
-    v4i w[D][2][2], x[D][2][2];
-    auto load_w = [&](v4i (&d)[2][2], int i) {
+    v4i w[D][FB][2], x[D][2][2];
+    auto load_w = [&](v4i (&d)[FB][2], int i) {
       const int8_t* t = a.w8 + (int64_t)(first_p + min(i, cnt8 - 1) * W) * 4096;
 #pragma unroll
-      for (int f = 0; f < 2; ++f)
+      for (int f = 0; f < FB; ++f)
 #pragma unroll
         for (int h = 0; h < 2; ++h) d[f][h] = *reinterpret_cast<const v4i*>(t + woff[f] + h * wh);
     };
@@ -647,11 +685,11 @@ gemm_prefill_split_kernel(PrefillArgs a) {
 #pragma unroll
       for (int d = 0; d < D; ++d) {
         const int i = i0 + d, in = i + D;
-        // tile i's operands: the 8 loads of each of the D - 1 tiles after it
+        // tile i's operands: the loads of each of the D - 1 tiles after it
         // may stay in flight (waiting here, outside the branch, keeps the
         // compiler from waiting for everything)
         if constexpr (DUMP) wait_vmcnt<0>();
-        else wait_vmcnt<8 * (D - 1)>();
+        else wait_vmcnt<(2 * FB + 4) * (D - 1)>();
         if (i < cnt8) {
           if (i > 0 && (i & 63) == 0) {
             wc = wcn;
@@ -660,10 +698,10 @@ gemm_prefill_split_kernel(PrefillArgs a) {
           }
           const float sc = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(wsc), i & 63));
           const int p = first_p + i * W;
-          tile_mac<2>(
+          tile_mac<FB, 2>(
               acc, w[d], x[d], sc, [](int) {},
               [&](int f, int t, const v16i& m) {
-                if constexpr (DUMP) dump_block(a, p, n0 + 32 * t, 32 * f, lane, m);
+                if constexpr (DUMP) dump_block(a, p, n0 + 32 * t, f0 + 32 * f, lane, m);
               });
         }
         __builtin_amdgcn_sched_barrier(0);
@@ -677,76 +715,39 @@ gemm_prefill_split_kernel(PrefillArgs a) {
     wait_vmcnt<0>();
   }
 
-  int8_t* region = lds + wave * kPdRegion;
-  if (a.w16 != nullptr) {
-    const int lo16r = a.rp16[r], n16r = a.rp16[r + 1] - lo16r;
-    const int f16 = (wave - n8r % W + W) % W;
-    const int cnt16 = n16r > f16 ? (n16r - f16 + W - 1) / W : 0;
-    const int first_q = lo16r + f16;
-    const int xch = ((lane & 7) ^ (lane >> 3)) * 8;
-    auto fetch_x16 = [&](int c) {          // 64 rows of 128 bytes, 16-byte chunk c of row R at slot c ^ (R % 8)
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const int64_t row = min(n0 + 8 * i + (lane >> 3), a.n - 1);
-        dma16(a.xf + row * a.ldx + c * 64 + xch, region + i * 1024);
-      }
-    };
-    int woff[2];
-#pragma unroll
-    for (int f = 0; f < 2; ++f)
-      woff[f] = a.layout == TQ_LAYOUT_MFMA ? (2 * f + rowpart) * 1024 + kpart * 128 + j * 8
-                                           : (f * 32 + (lane & 31)) * 64 + kpart * 8;
-    v4i w[2][4];
-    auto load_w16 = [&](int q) {
-      const uint16_t* t = a.w16 + (int64_t)q * 4096;
-#pragma unroll
-      for (int f = 0; f < 2; ++f)
-#pragma unroll
-        for (int kc = 0; kc < 4; ++kc)
-          w[f][kc] = *reinterpret_cast<const v4i*>(
-              t + woff[f] + (a.layout == TQ_LAYOUT_MFMA ? (kc >> 1) * 512 + (kc & 1) * 256 : kc * 16));
-    };
-    uint32_t xrd[4];
-#pragma unroll
-    for (int kc = 0; kc < 4; ++kc)
-      xrd[kc] = lds_addr(region) + (lane & 31) * 128 + (((2 * kc + kpart) ^ (lane & 7)) * 16);
-    for (int w0 = 0; w0 < cnt16; w0 += 64) {
-      const int cols = col_of(a.ids16[first_q + min(w0 + lane, cnt16 - 1) * W], r * n_tc, n_tc);
-      const int nq = min(64, cnt16 - w0);
-      fetch_x16(__builtin_amdgcn_readlane(cols, 0));
-      load_w16(first_q + w0 * W);
-      for (int i = 0; i < nq; ++i) {
-        const int in = min(i + 1, nq - 1);
-        wait_vmcnt<0>();
-        v4i xv[2][4];
-        asm volatile(
-            "ds_read_b128 %0, %8\n\t"
-            "ds_read_b128 %1, %9\n\t"
-            "ds_read_b128 %2, %10\n\t"
-            "ds_read_b128 %3, %11\n\t"
-            "ds_read_b128 %4, %8 offset:4096\n\t"
-            "ds_read_b128 %5, %9 offset:4096\n\t"
-            "ds_read_b128 %6, %10 offset:4096\n\t"
-            "ds_read_b128 %7, %11 offset:4096\n\t"
-            "s_waitcnt lgkmcnt(0)"
-            : "=&v"(xv[0][0]), "=&v"(xv[0][1]), "=&v"(xv[0][2]), "=&v"(xv[0][3]), "=&v"(xv[1][0]), "=&v"(xv[1][1]),
-              "=&v"(xv[1][2]), "=&v"(xv[1][3])
-            : "v"(xrd[0]), "v"(xrd[1]), "v"(xrd[2]), "v"(xrd[3])
-            : "memory");
-        __builtin_amdgcn_sched_barrier(0);
-        fetch_x16(__builtin_amdgcn_readlane(cols, in));   // the operands are in registers: refill at once
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int kc = 0; kc < 4; ++kc)
-#pragma unroll
-          for (int t = 0; t < 2; ++t)
-#pragma unroll
-            for (int f = 0; f < 2; ++f) acc[f][t] = mfma32<XT>(w[f][kc], xv[t][kc], acc[f][t]);
-        __builtin_amdgcn_sched_barrier(0);
-        load_w16(first_q + (w0 + in) * W);
-        __builtin_amdgcn_sched_barrier(0);
-      }
+  if (cnt16 > 0) {
+    const uint32_t xrd0 = lds_addr(region) + (lane & 31) * 128;
+    const uint32_t wrd = lds_addr(region) + 8192 + rowpart * 2048 + kpart * 256 + j * 16;
+    for (int i = 0; i < cnt16; ++i) {
       wait_vmcnt<0>();
+#pragma unroll
+      for (int kc = 0; kc < 4; ++kc) {     // 16-deep slices, in order
+        const uint32_t xrd = xrd0 + (((2 * kc + kpart) ^ (lane & 7)) * 16);
+        const uint32_t wr = wrd + (kc >> 1) * 1024 + (kc & 1) * 512;
+        v4i xv[2], wv[FB];
+        asm volatile(
+            "ds_read_b128 %0, %3\n\t"
+            "ds_read_b128 %1, %3 offset:4096\n\t"
+            "ds_read_b128 %2, %4\n\t"
+            "s_waitcnt lgkmcnt(0)"
+            : "=&v"(xv[0]), "=&v"(xv[1]), "=&v"(wv[0])
+            : "v"(xrd), "v"(wr)
+            : "memory");
+        if constexpr (FB == 2)
+          asm volatile("ds_read_b128 %0, %1 offset:4096\n\ts_waitcnt lgkmcnt(0)"
+                       : "=&v"(wv[FB - 1])
+                       : "v"(wr)
+                       : "memory");
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+          for (int f = 0; f < FB; ++f) acc[f][t] = mfma32<XT>(wv[f], xv[t], acc[f][t]);
+      }
+      if (i + 1 < cnt16) {                 // every operand is in registers: refill
+        if (((i + 1) & 63) == 0) wcol16 = cols16(i + 1);
+        __builtin_amdgcn_sched_barrier(0);
+        fetch16(first_q + (i + 1) * W, __builtin_amdgcn_readlane(wcol16, (i + 1) & 63));
+      }
     }
   }
 
@@ -770,36 +771,32 @@ gemm_prefill_split_kernel(PrefillArgs a) {
     else go(TypeTag<Fp16>{});
     return o;
   };
-  {
-    // Partial sums through LDS, one 32-feature half at a time: chunk
-    // (t, g) of wave w is 64 lanes x 4 features, summed over the waves in
-    // wave order by wave (chunk % W).
-    int8_t* staged = lds + W * kPdRegion;
+  // Partial sums through LDS: chunk (f, t, g) of wave w is 64 lanes x 4
+  // features, summed over the waves in wave order by wave (chunk % W); the
+  // rounded outputs are staged and leave as 128-byte rows.
+  int8_t* staged = lds + W * kPdRegion;
 #pragma unroll
-    for (int f = 0; f < 2; ++f) {
-      __syncthreads();   // the regions are free (16-bit operands read; the previous half summed)
+  for (int f = 0; f < FB; ++f)
 #pragma unroll
-      for (int t = 0; t < 2; ++t)
+    for (int t = 0; t < 2; ++t)
 #pragma unroll
-        for (int g = 0; g < 4; ++g)
-          *reinterpret_cast<v4f*>(region + (t * 4 + g) * 1024 + lane * 16) =
-              v4f{acc[f][t][4 * g], acc[f][t][4 * g + 1], acc[f][t][4 * g + 2], acc[f][t][4 * g + 3]};
-      __syncthreads();
-      for (int q = wave; q < 8; q += W) {
-        v4f s = *reinterpret_cast<const v4f*>(lds + q * 1024 + lane * 16);
-        for (int u = 1; u < W; ++u) {
-          const v4f b = *reinterpret_cast<const v4f*>(lds + u * kPdRegion + q * 1024 + lane * 16);
+      for (int g = 0; g < 4; ++g)
+        *reinterpret_cast<v4f*>(region + (f * 8 + t * 4 + g) * 1024 + lane * 16) =
+            v4f{acc[f][t][4 * g], acc[f][t][4 * g + 1], acc[f][t][4 * g + 2], acc[f][t][4 * g + 3]};
+  __syncthreads();
+  for (int q = wave; q < 8 * FB; q += W) {
+    v4f s = *reinterpret_cast<const v4f*>(lds + q * 1024 + lane * 16);
+    for (int u = 1; u < W; ++u) {
+      const v4f p = *reinterpret_cast<const v4f*>(lds + u * kPdRegion + q * 1024 + lane * 16);
 #pragma unroll
-          for (int e = 0; e < 4; ++e) s[e] += b[e];
-        }
-        const int t = q >> 2, g = q & 3, row = t * 32 + (lane & 31), feat = f * 32 + 8 * g + 4 * kpart;
-        const float y[4] = {s[0], s[1], s[2], s[3]};
-        *reinterpret_cast<u32x2*>(staged + row * 128 + (((f * 4 + g) ^ (row & 7)) * 16) + kpart * 8) = round4(y, feat);
-      }
+      for (int e = 0; e < 4; ++e) s[e] += p[e];
     }
-    __syncthreads();
-    store_rows(a, staged, r, n0, 64, threadIdx.x, blockDim.x);
+    const int f = q >> 3, t = (q >> 2) & 1, g = q & 3, row = t * 32 + (lane & 31), feat = f0 + f * 32 + 8 * g + 4 * kpart;
+    const float y[4] = {s[0], s[1], s[2], s[3]};
+    *reinterpret_cast<u32x2*>(staged + row * 128 + (((f0 / 8 + f * 4 + g) ^ (row & 7)) * 16) + kpart * 8) = round4(y, feat);
   }
+  __syncthreads();
+  store_rows<4 * FB>(a, staged, r, n0, 64, threadIdx.x, blockDim.x, f0 / 8);
 }
 
 }  // namespace tq
@@ -812,16 +809,16 @@ using namespace tq;
 //
 // Split lists while whole-list workgroups leave most of the chip waiting for
 // each wave's serial walk (0.56 us per tile).  Measured on MI355X, us per launch,
-// whole list -> split over 4 waves, 96 / 192 / 384 / 512 tokens:
-//   Llama-3.2-3B Q/K/V   32 -> 14   33 -> 14   33 -> 19   34 -> 27
-//     O                  33 -> 13   33 -> 14   33 -> 18   33 -> 18
-//     Gate/Up            35 -> 20   35 -> 31   47 -> 49   50 -> 63
-//   Qwen2.5-7B Gate/Up   56 -> 55   90 -> 74   96 -> 130  142 -> 179
+// whole list -> split over 4 waves, 128 / 192 / 384 / 512 tokens:
+//   Llama-3.2-3B Q/K/V   35 -> 15   35 -> 15   35 -> 20   34 -> 27
+//     O                  33 -> 10   32 -> 13   33 -> 16   33 -> 18
+//     Gate/Up            38 -> 24   38 -> 33   48 -> 51   50 -> 63
+//   Qwen2.5-7B Gate/Up   56 -> 54   90 -> 70   96 -> 125  142 -> 179
 // so the layer's three together gain up to about 400 tokens.  Long lists (Down)
-// longer, 192 / 1024 / 1500 tokens: Llama 73 -> 23, 77 -> 54, 103 -> 87;
-// Qwen2.5-7B 160 -> 44, 173 -> 139, 229 -> 219; 14B 120 -> 36, 173 -> 131, 183 ->
-// 221.  Eight waves where the list is long and the grid small (192 tokens: 21,
-// 38 and 32 against 23, 44 and 36 us; at 384 37, 71, 59 against 32, 64, 53).
+// longer, 192 / 1024 / 1500 tokens: Llama 80 -> 26, 77 -> 54, 103 -> 87;
+// Qwen2.5-7B 174 -> 51, 173 -> 139, 229 -> 219; 14B 131 -> 41, 173 -> 131, 183 ->
+// 221.  Eight waves where the list is long and the grid small (192 tokens: 24,
+// 46 and 39 against 26, 51 and 41 us; at 384 39, 84, 67 against 34, 76, 63).
 constexpr int kSplitTokens = 384, kSplitLongTokens = 1280, kSplitLongTiles = 96, kSplitWideTokens = 256;
 static int split_waves(int n, int n_tc) {
   if (n > (n_tc >= kSplitLongTiles ? kSplitLongTokens : kSplitTokens)) return 0;
@@ -847,17 +844,30 @@ static int blocked_tb(int n, int units) {
   return (l4 / 2) * 83 + (l4 % 2) * 55 < (l2 / 3) * 68 + rest2[l2 % 3] ? 4 : 2;
 }
 
+// Half row tiles while the whole ones leave half of the CUs without work (the
+// same sums).  Measured on MI355X with cold weights, whole -> half (us): Llama O
+// (48 row tiles) at 128 tokens 12.7 -> 9.7, at 192 12.7 -> 11.6; Down (eight waves)
+// at 128 24.9 -> 19.2, at 192 24.5 -> 28.9; Qwen2.5-7B Down (56) at 128 47.4 ->
+// 36.9, at 192 46.5 -> 64.4; Q/K/V (80) at 128 14.9 -> 15.9.
+constexpr int kSplitHalfGrid = 128;
+static bool split_halves(int n, int n_tr) { return (int64_t)n_tr * ((n + 63) / 64) <= kSplitHalfGrid; }
+
+template <class XT, int FB, bool DUMP>
+static hipError_t launch_split(const PrefillArgs& a, int W, hipStream_t s) {
+  constexpr auto kern = gemm_prefill_split_kernel<XT, FB, kPdAhead, DUMP>;
+  const int64_t blocks = 8ll * ((a.n_tr + 7) / 8) * ((a.n + 63) / 64) * (2 / FB);
+  if (blocks >= (1ll << 31)) return hipErrorInvalidValue;
+  const size_t lds = (size_t)W * kPdRegion + 8192;
+  const hipError_t e = allow_lds<kern>(lds);
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(64 * W), lds, s, a);
+  return hipGetLastError();
+}
+
 template <class XT, bool DUMP>
 static hipError_t launch_blocked(PrefillArgs a, hipStream_t s) {
   if (const int W = split_waves(a.n, a.n_tc)) {
-    constexpr auto kern = gemm_prefill_split_kernel<XT, 2, DUMP>;
-    const int64_t blocks = 8ll * ((a.n_tr + 7) / 8) * ((a.n + 63) / 64);
-    if (blocks >= (1ll << 31)) return hipErrorInvalidValue;
-    const size_t lds = (size_t)W * kPdRegion + 8192;
-    const hipError_t e = allow_lds<kern>(lds);
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(64 * W), lds, s, a);
-    return hipGetLastError();
+    return split_halves(a.n, a.n_tr) ? launch_split<XT, 1, DUMP>(a, W, s) : launch_split<XT, 2, DUMP>(a, W, s);
   }
   a.n_units = (a.n_slots + 3) / 4;
   const int tb = blocked_tb(a.n, a.n_units);
