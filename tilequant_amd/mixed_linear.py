@@ -99,10 +99,7 @@ def _view_key(t: torch.Tensor) -> Tuple[Any, ...]:
     """What makes two uses of a tensor see the same values: its storage view
     and its version counter (inference tensors have none; they cannot be
     modified in place outside inference mode either)."""
-    try:
-        version = int(t._version)
-    except RuntimeError:
-        version = None
+    version = None if t.is_inference() else int(t._version)
     return (t.data_ptr(), t.storage_offset(), tuple(t.shape), tuple(t.stride()), t.dtype, t.device, version)
 
 
@@ -335,11 +332,11 @@ class MixedLinear(nn.Module):
             prefill_plan=self._prefill_plan(int(x_fp.shape[0])), x_int8_layout=x_int8_layout,
         )
 
-    def _prompt_blocked(self, n_rows: int, x_work: torch.Tensor) -> bool:
+    def _prompt_blocked(self, x_work: torch.Tensor) -> bool:
         """Whether a prompt-size input runs on token-blocked codes
         (``gemm_mixed_rows_blocked``): full column tiles, aligned rows.  The
         other inputs (and those taken in row chunks) keep row-major codes."""
-        return (n_rows > PLAN_MIN_ROWS and self.tile_n == 64 and self.K_orig == 64 * self.n_tc
+        return (self.tile_n == 64 and self.K_orig == 64 * self.n_tc
                 and 1 <= self.n_tc <= BLOCKED_MAX_COLUMN_TILES and x_work.is_cuda and _blockable(x_work))
 
     def _build_prompt(self, x_work: torch.Tensor, out_dtype: torch.dtype, order: Optional[torch.Tensor]) -> _Launch:
@@ -561,10 +558,10 @@ class MixedLinear(nn.Module):
             y = self._cached_forward(x_work)
             return y.reshape(in_shape[0], in_shape[1], self.M_orig) if x.dim() == 3 else y
         chunk = self._activation_row_chunk_size()
-        if 0 < n_rows <= min(self._fused_rows_for_cfg(), chunk):
-            y = self._fused_decode(x_work)
-        elif n_rows <= chunk and self._prompt_blocked(n_rows, x_work):
+        if PLAN_MIN_ROWS < n_rows <= chunk and self._prompt_blocked(x_work):   # above every fused launch's rows
             y = self._prompt_forward(x, x_work)
+        elif 0 < n_rows <= min(self._fused_rows_for_cfg(), chunk):
+            y = self._fused_decode(x_work)
         elif n_rows <= chunk:
             blocked = self.token_blocked_codes(n_rows) and _blockable(x_work)
             x_int8, sx = _quantize_for(self, x, x_work, blocked)
