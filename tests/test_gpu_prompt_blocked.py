@@ -75,6 +75,8 @@ def test_blocked_quantizer_matches_the_oracle(n, dtype):
     (513, 704, 4160, 0.3, torch.bfloat16, "mfma", True),       # 65 column tiles: two windows, an odd count
     (1000, 8192, 320, 0.1, torch.bfloat16, "row_major", True),
     (2049, 16384, 128, 0.1, torch.float16, "mfma", False),     # 128-token workgroups
+    (2100, 16384, 192, 0.2, torch.bfloat16, "mfma", False),    # the last one with 52 tokens: half of its blocks
+    (2052, 16384, 256, 0.1, torch.bfloat16, "mfma", True),     # a short last one beside row tiles in 16 bits
     (1281, 192, 8192, 0.1, torch.bfloat16, "mfma", False),     # long lists past the split limit
     (1300, 128, 19456, 0.05, torch.bfloat16, "mfma", False),   # the most column tiles it takes
 ])

@@ -143,8 +143,11 @@ __device__ inline void store_rows(const PrefillArgs& a, const int8_t* staged, in
 // against 41%), and token-blocked slices cross the LDS DMA path at twice the
 // rate of row-major ones (probe of the loads alone: 25 against 12 TB/s).  Per
 // Llama-3.2-3B layer (keep05, quantization included) against the row-major
-// kernel: 2048 tokens 558 -> 418 us, 8192 tokens 1537 -> 1383 us; Qwen2.5-7B
-// (clustered keep10, fp16) at 777 tokens 827 -> 539 us.
+// kernel: 2048 tokens 558 -> 424 us, 8192 tokens 1537 -> 1383 us; Qwen2.5-7B
+// (clustered keep10, fp16) at 777 tokens 826 -> 488 us.
+//
+// NT <= TB: the 32-token blocks that a wave multiplies, fewer in a short last
+// workgroup (the loads stay, so the waits count the same).
 // 16-bit phase: see there.  Outputs are staged in the wave's quarter of the
 // ring and leave as 128-byte rows.
 constexpr int kPbCols = 304;     // column tiles (k <= 19456)
@@ -165,7 +168,7 @@ struct BlockedLds {
   int n_cols16;
 };
 
-template <class XT, int TB, bool SHARED16, bool DUMP>
+template <class XT, int TB, int NT, bool SHARED16, bool DUMP>
 __device__ __attribute__((always_inline)) inline void prefill_blocked_body(const PrefillArgs& a, BlockedLds<TB>& lds,
                                                                            const SlotTiles& tiles, int n0, bool any8,
                                                                            int lane, int wave) {
@@ -178,11 +181,11 @@ __device__ __attribute__((always_inline)) inline void prefill_blocked_body(const
   const int r = tiles.r, lo8 = tiles.lo8, hi8 = tiles.hi8, lo16 = tiles.lo16, hi16 = tiles.hi16;
   const int last8 = a.rp8[a.n_tr] - 1;     // any8: at least 0
 
-  v16f acc[2][TB];
+  v16f acc[2][NT];
 #pragma unroll
   for (int f = 0; f < 2; ++f)
 #pragma unroll
-    for (int t = 0; t < TB; ++t)
+    for (int t = 0; t < NT; ++t)
 #pragma unroll
       for (int v = 0; v < 16; ++v) acc[f][t][v] = 0.f;
 
@@ -250,40 +253,24 @@ __device__ __attribute__((always_inline)) inline void prefill_blocked_body(const
       if ((mask >> i) & 1) {
         const float sc = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(wsc), i));
         const uint32_t rd = x_rd + (s % kPbStages) * XB;
-        v4i x[TB][2];
-        if constexpr (TB == 4) {
+        v4i x[NT][2];
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
           asm volatile(
-              "ds_read_b128 %0, %8\n\t"
-              "ds_read_b128 %1, %8 offset:512\n\t"
-              "ds_read_b128 %2, %8 offset:2048\n\t"
-              "ds_read_b128 %3, %8 offset:2560\n\t"
-              "ds_read_b128 %4, %8 offset:4096\n\t"
-              "ds_read_b128 %5, %8 offset:4608\n\t"
-              "ds_read_b128 %6, %8 offset:6144\n\t"
-              "ds_read_b128 %7, %8 offset:6656\n\t"
-              : "=&v"(x[0][0]), "=&v"(x[0][1]), "=&v"(x[1][0]), "=&v"(x[1][1]), "=&v"(x[TB - 2][0]),
-                "=&v"(x[TB - 2][1]), "=&v"(x[TB - 1][0]), "=&v"(x[TB - 1][1])
-              : "v"(rd)
+              "ds_read_b128 %0, %2 offset:%3\n\t"
+              "ds_read_b128 %1, %2 offset:%4"
+              : "=&v"(x[t][0]), "=&v"(x[t][1])
+              : "v"(rd), "n"(2048 * t), "n"(2048 * t + 512)
               : "memory");
-        } else {
-          asm volatile(
-              "ds_read_b128 %0, %4\n\t"
-              "ds_read_b128 %1, %4 offset:512\n\t"
-              "ds_read_b128 %2, %4 offset:2048\n\t"
-              "ds_read_b128 %3, %4 offset:2560\n\t"
-              : "=&v"(x[0][0]), "=&v"(x[0][1]), "=&v"(x[1][0]), "=&v"(x[1][1])
-              : "v"(rd)
-              : "memory");
-        }
         const int p = DUMP ? pw[s] : 0;
-        tile_mac<2, TB>(
+        tile_mac<2, NT>(
             acc, ws, x, sc,
             [&](int t) {
               // LDS reads return in order: token block t has landed when at
-              // most 2 (TB - 1 - t) reads are outstanding
-              if (t == TB - 1 || DUMP) asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(x[t][0]), "+v"(x[t][1])::"memory");
-              else if (t == TB - 2) asm volatile("s_waitcnt lgkmcnt(2)" : "+v"(x[t][0]), "+v"(x[t][1])::"memory");
-              else if (t == TB - 3) asm volatile("s_waitcnt lgkmcnt(4)" : "+v"(x[t][0]), "+v"(x[t][1])::"memory");
+              // most 2 (NT - 1 - t) reads are outstanding
+              if (t == NT - 1 || DUMP) asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(x[t][0]), "+v"(x[t][1])::"memory");
+              else if (t == NT - 2) asm volatile("s_waitcnt lgkmcnt(2)" : "+v"(x[t][0]), "+v"(x[t][1])::"memory");
+              else if (t == NT - 3) asm volatile("s_waitcnt lgkmcnt(4)" : "+v"(x[t][0]), "+v"(x[t][1])::"memory");
               else asm volatile("s_waitcnt lgkmcnt(6)" : "+v"(x[t][0]), "+v"(x[t][1])::"memory");
             },
             [&](int f, int t, const v16i& d) {
@@ -420,11 +407,9 @@ __device__ __attribute__((always_inline)) inline void prefill_blocked_body(const
         if (__builtin_amdgcn_readlane(eq, i) >= 0 && e < nc) {
           const uint32_t base = lds_addr(ring) + (e & 3) * SB;
           block_mfma(ws, base, std::integral_constant<int, 0>{});
-          block_mfma(ws, base + 4096, std::integral_constant<int, 1>{});
-          if constexpr (TB == 4) {
-            block_mfma(ws, base + 8192, std::integral_constant<int, TB - 2>{});
-            block_mfma(ws, base + 12288, std::integral_constant<int, TB - 1>{});
-          }
+          if constexpr (NT > 1) block_mfma(ws, base + 4096, std::integral_constant<int, 1>{});
+          if constexpr (NT > 2) block_mfma(ws, base + 8192, std::integral_constant<int, 2>{});
+          if constexpr (NT > 3) block_mfma(ws, base + 12288, std::integral_constant<int, 3>{});
         }
         __builtin_amdgcn_sched_barrier(0);
         load_w16(ws, min(max(__builtin_amdgcn_readlane(eqn, i), 0), last16));
@@ -453,8 +438,9 @@ __device__ __attribute__((always_inline)) inline void prefill_blocked_body(const
       };
       auto half_mfma = [&](const v4i (&ws)[2][4], auto half_tag) {
         constexpr int H = decltype(half_tag)::value;
-        block_mfma(ws, rd + H * kHalf, std::integral_constant<int, H * (TB / 2)>{});
-        if constexpr (TB == 4) block_mfma(ws, rd + H * kHalf + 4096, std::integral_constant<int, H * (TB / 2) + TB / 2 - 1>{});
+        constexpr int t = H * (TB / 2);
+        if constexpr (t < NT) block_mfma(ws, rd + H * kHalf, std::integral_constant<int, t>{});
+        if constexpr (TB == 4 && t + 1 < NT) block_mfma(ws, rd + H * kHalf + 4096, std::integral_constant<int, t + 1>{});
       };
       for (int q0 = lo16; q0 < hi16; q0 += 64) {
         const int cols = col_of(a.ids16[min(q0 + lane, hi16 - 1)], r * n_tc, n_tc);
@@ -499,7 +485,7 @@ __device__ __attribute__((always_inline)) inline void prefill_blocked_body(const
 #pragma unroll
           for (int e = 0; e < 4; ++e) bv[e] = OT::to_f32(a.bias[min(r * 64 + feat + e, a.m - 1)]);
 #pragma unroll
-        for (int t = 0; t < TB; ++t) {
+        for (int t = 0; t < NT; ++t) {
           const int row = t * 32 + (lane & 31);
           u32x2 y;
 #pragma unroll
@@ -521,7 +507,7 @@ __device__ __attribute__((always_inline)) inline void prefill_blocked_body(const
     else stage_out(TypeTag<Fp16>{}, std::false_type{});
   }
   __builtin_amdgcn_s_waitcnt(0xC07F);   // lgkmcnt(0): the wave reads back only its own rows
-  store_rows(a, region, r, n0, 32 * TB, lane, 64);
+  store_rows(a, region, r, n0, 32 * NT, lane, 64);
 }
 
 template <class XT, int TB, bool DUMP = false>
@@ -550,8 +536,16 @@ gemm_prefill_blocked_kernel(PrefillArgs a) {
   const SlotTiles mine{of_wave(rv), of_wave(lo8v), of_wave(hi8v), of_wave(lo16v), of_wave(hi16v), of_wave(okv) != 0};
   // Row tiles mostly in 16 bits: the waves share the activation slices of the
   // 16-bit phase too (two programs, so that neither pays the other's registers).
-  if (heavy) prefill_blocked_body<XT, TB, true, DUMP>(a, lds, mine, n0, any8, lane, wave);
-  else prefill_blocked_body<XT, TB, false, DUMP>(a, lds, mine, n0, any8, lane, wave);
+  // A last workgroup of few tokens multiplies only the blocks it has (1, 2 or 4 of
+  // them); it is dispatched last and fills the last wave of the grid.  Measured
+  // on MI355X, cold weights, all blocks -> these: Qwen2.5-7B Gate/Up at 777
+  // tokens (9 of 128 in the last) 220 -> 201 us, at 1030 279 -> 258;
+  // Llama-3.2-3B Gate/Up at 1030 119 -> 97; Qwen2.5-7B O at 777 40 -> 38.
+  const int left = a.n - n0;
+  if (heavy) prefill_blocked_body<XT, TB, TB, true, DUMP>(a, lds, mine, n0, any8, lane, wave);
+  else if (left > 16 * TB) prefill_blocked_body<XT, TB, TB, false, DUMP>(a, lds, mine, n0, any8, lane, wave);
+  else if (TB == 4 && left > 32) prefill_blocked_body<XT, TB, TB / 2, false, DUMP>(a, lds, mine, n0, any8, lane, wave);
+  else prefill_blocked_body<XT, TB, 1, false, DUMP>(a, lds, mine, n0, any8, lane, wave);
 }
 
 // ---- few tokens: the row tile's list split over the waves of a workgroup ------
