@@ -1,6 +1,12 @@
 """Host logic of the prompt GEMM (no GPU): the slot order of a weight's row tiles."""
 from __future__ import annotations
 
+import os
+import re
+import struct
+import subprocess
+from pathlib import Path
+
 import numpy as np
 import pytest
 
@@ -54,3 +60,70 @@ def test_prompt_entries_reject_bad_arguments_before_any_launch():
         assert lib.tq_gemm_mixed_blocked(*bad) == code, (at, value)
     assert lib.tq_gemm_mixed_blocked(*[fake if i == 22 else a for i, a in enumerate(args)]) == -1   # no slots
     assert lib.tq_prompt_forward(None) == -1
+
+
+def _blocked_kernel_listings(tmp_path):
+    """{symbol: instructions} of the whole-list prompt kernels in the library
+    built from this tree (its gfx950 code objects, listed by llvm-objdump)."""
+    llvm = Path(os.environ.get("ROCM_PATH", "/opt/rocm")) / "llvm" / "bin"
+    fat = tmp_path / "fatbin"
+    subprocess.run([llvm / "llvm-objcopy", f"--dump-section=.hip_fatbin={fat}", nat.LIB_PATH, tmp_path / "rest"],
+                   check=True)
+    data, magic, listings = fat.read_bytes(), b"__CLANG_OFFLOAD_BUNDLE__", {}
+    for found in re.finditer(magic, data):
+        base, at = found.start(), found.end()
+        (entries,) = struct.unpack_from("<Q", data, at)
+        at += 8
+        for _ in range(entries):
+            offset, size, id_len = struct.unpack_from("<QQQ", data, at)
+            at += 24 + id_len
+            code = data[base + offset:base + offset + size]
+            if b"gfx950" not in data[at - id_len:at] or b"gemm_prefill_blocked_kernel" not in code:
+                continue
+            obj = tmp_path / "code.o"
+            obj.write_bytes(code)
+            text = subprocess.run([llvm / "llvm-objdump", "-d", "--no-show-raw-insn", obj], check=True,
+                                  capture_output=True, text=True).stdout
+            for part in re.split(r"\n(?=[0-9a-f]+ <[^>]+>:\n)", text):
+                head = re.match(r"([0-9a-f]+) <([^>]+)>:\n", part)
+                if head and "gemm_prefill_blocked_kernel" in head[2]:
+                    ins = re.findall(r"^\s+([a-z]\w+.*?)\s*//\s*([0-9A-F]+):", part, flags=re.M)
+                    listings[head[2]] = [(int(addr, 16), text) for text, addr in ins]
+    return listings
+
+
+@pytest.mark.skipif(not Path("/opt/rocm/llvm/bin/llvm-objdump").exists(), reason="no llvm-objdump")
+def test_ring_slices_land_before_the_first_barrier_publishes_them(tmp_path):
+    """The whole-list kernel's waves fill each LDS ring stage together, so a
+    wave's own loads of the first two slices must have landed before its first
+    ring barrier.  In the built code: after the prologue's 6 XL LDS loads (XL
+    per slice), the waits before that barrier leave in flight no more than the
+    vector memory operations issued after the first 2 XL."""
+    listings = _blocked_kernel_listings(tmp_path)
+    assert len(listings) == 6            # bf16 and fp16 x 64 and 128 tokens, and the bf16 dumps
+    for name, ins in listings.items():
+        xl = 2 if "ELi4E" in name else 1
+        index = {addr: i for i, (addr, _) in enumerate(ins)}
+        vmem = [bool(re.match(r"(global|buffer|flat)_", text)) for _, text in ins]
+        loads = [i for i, v in enumerate(vmem) if v]
+        bodies = 0
+        for first in range(len(loads)):
+            run = loads[first:first + 6 * xl + 1]
+            lds = ["_lds_" in ins[i][1] for i in run]
+            if first and "_lds_" in ins[loads[first - 1]][1] or lds != [True] * (6 * xl) + [False]:
+                continue
+            bodies += 1
+            i, since, landed, hops = run[2 * xl - 1] + 1, 0, False, 0
+            while not ins[i][1].startswith("s_barrier"):
+                text = ins[i][1]
+                since += vmem[i]
+                wait = re.match(r"s_waitcnt.*vmcnt\((\d+)\)", text)
+                landed = landed or bool(wait) and int(wait[1]) <= since
+                jump = re.match(r"s_branch (\S+)", text)
+                i += 1
+                if jump:
+                    hops += 1
+                    assert hops < 20, name
+                    i = index[ins[i - 1][0] + 4 + 4 * ((int(jump[1], 0) + 0x8000) % 0x10000 - 0x8000)]
+            assert landed, f"{name}: the first ring barrier is passed with {since} later operations and no wait"
+        assert bodies >= 3, name         # 1, 2 or 4 token blocks, and the 16-bit-heavy row tiles

@@ -213,6 +213,7 @@ __device__ __attribute__((always_inline)) inline void prefill_blocked_body(const
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
 #pragma unroll
     for (int s = 0; s < 2 * kPbAhead; ++s) fetch_x(s);
+    __builtin_amdgcn_sched_barrier(0);
 
     // weight operand (feature block f, K half h) of this lane inside a tile
     int woff[2];
@@ -235,6 +236,11 @@ __device__ __attribute__((always_inline)) inline void prefill_blocked_body(const
     __builtin_amdgcn_sched_barrier(0);
     load_w(w[1], __builtin_amdgcn_readfirstlane(p1));
     __builtin_amdgcn_sched_barrier(0);
+    // The wave's share of slices 0 and 1 lands before the first barrier, past
+    // which the other waves read it: only the later slices' fetches and both
+    // steps' weights (2 x 4 loads) may stay in flight.
+    if constexpr (DUMP) wait_vmcnt<0>();
+    else wait_vmcnt<(2 * kPbAhead - 2) * XL + 8>();
 
     const uint32_t x_rd = lds_addr(ring) + ((lane >> 4) & 1) * 1024 + (lane >> 5) * 256 + (lane & 15) * 16;
     // window of 64 columns: lane i holds column c0 + i's scale and the
@@ -284,11 +290,13 @@ __device__ __attribute__((always_inline)) inline void prefill_blocked_body(const
     const int iters = (n_tc + 1) / 2;
     for (int k = 0; k < iters; ++k) {
       const int s = 2 * k;
-      // Slices s and s + 1 were fetched kPbAhead iterations ago; the two
-      // iterations since issued at least 2 (2 XL + 8) vector memory
-      // operations, which complete in order.  Past the barrier every wave is
-      // done with the stages of the previous iteration, which the fetch below
-      // reuses.
+      // The wave's share of slices s and s + 1 has landed before the barrier
+      // (vector memory operations complete in order): for k = 0 by the wait
+      // above, for the prologue's other slices by the waits of the steps of
+      // k = 0, and from k = kPbAhead on, fetched kPbAhead iterations ago, by
+      // this one, as the two iterations since issued 2 (2 XL + 8) operations
+      // after them.  Past the barrier every wave is done with the stages of
+      // the previous iteration, which the fetch below reuses.
       if constexpr (DUMP) wait_vmcnt<0>();
       else wait_vmcnt<2 * (2 * XL + 8)>();
       asm volatile("s_barrier" ::: "memory");
