@@ -1,0 +1,115 @@
+"""Host logic of the activation codes that sibling projections share (no GPU):
+``MixedLinear._prompt_forward`` against a stand-in for the foreign call, whose
+"quantizer" writes the input's first value at the head of the codes and whose
+"GEMM" writes the head of the codes it is given to the output's first value."""
+from __future__ import annotations
+
+import ctypes
+from types import SimpleNamespace
+
+import pytest
+import torch
+
+from test_host_logic import _cpu_pack
+from tilequant_amd import mixed_linear as ml
+from tilequant_amd.mixed_linear import MixedLinear
+
+CFG = SimpleNamespace(dtype_out="bf16")
+ROWS, COLS = 100, 192
+
+
+class _Library:
+    """Stands in for the foreign calls; ``before`` runs ahead of the launches
+    and returns the call's code."""
+
+    def __init__(self):
+        self.quantized = []
+        self.before = lambda: 0
+
+    def tq_prompt_forward(self, ref):
+        d = ref._obj
+        rc = self.before()
+        if rc:
+            return rc
+        self.quantized.append(bool(d.quantize))
+        if d.quantize:
+            ctypes.memmove(d.x_blocked, d.x, 2)
+        ctypes.memmove(d.out, d.x_blocked, 2)
+        return 0
+
+    @staticmethod
+    def tq_error_string(code):
+        return b"forced by the test"
+
+
+@pytest.fixture
+def library(monkeypatch):
+    lib = _Library()
+    monkeypatch.setattr(ml.nat, "lib", lambda: lib)
+    monkeypatch.setattr(ml.nat, "require_device", lambda *tensors: None)
+    monkeypatch.setattr(torch._C, "_cuda_getCurrentRawStream", lambda index: 0)
+    monkeypatch.setattr(ml, "_SHARED_QUANT", {})
+    return lib
+
+
+def _siblings(count=2):
+    return [MixedLinear(_cpu_pack(128, COLS, 0.3, seed)[0], None, CFG) for seed in range(count)]
+
+
+def _input(value):
+    return torch.full((ROWS, COLS), float(value), dtype=torch.bfloat16)
+
+
+def _call(lin, x):
+    return float(lin._prompt_forward(x, x)[0, 0])
+
+
+def test_siblings_share_one_quantization(library):
+    a, b = _siblings()
+    x = _input(2)
+    with torch.inference_mode():
+        assert [_call(a, x), _call(b, x), _call(a, x)] == [2, 2, 2]
+    assert library.quantized == [True, False, True]      # a consumer asking twice starts a new pass
+
+
+def test_codes_of_a_failed_call_are_not_shared(library, monkeypatch):
+    a, b = _siblings()
+    x = _input(3)
+    with torch.inference_mode():
+        library.before = lambda: 2
+        with pytest.raises(RuntimeError, match="forced"):
+            _call(a, x)
+        library.before = lambda: 0
+        assert _call(b, x) == 3
+
+        real = torch.empty
+
+        def no_room_for_the_output(size, *args, **kwargs):
+            if tuple(size) == (ROWS, 128):
+                raise torch.OutOfMemoryError("forced by the test")
+            return real(size, *args, **kwargs)
+
+        y = _input(4)
+        monkeypatch.setattr(torch, "empty", no_room_for_the_output)
+        with pytest.raises(torch.OutOfMemoryError):
+            _call(a, y)
+        monkeypatch.setattr(torch, "empty", real)
+        assert _call(b, y) == 4
+    assert library.quantized == [True, True]
+
+
+def test_codes_are_not_shared_before_their_launch(library):
+    """A second thread on the same stream, with the same input, while the first
+    is inside the foreign call and has launched nothing yet."""
+    a, b = _siblings()
+    x, seen = _input(5), []
+
+    def other_thread():
+        library.before = lambda: 0
+        seen.append(_call(b, x))
+        return 0
+
+    with torch.inference_mode():
+        library.before = other_thread
+        assert _call(a, x) == 5
+    assert seen == [5] and library.quantized == [True, True]

@@ -406,8 +406,6 @@ class MixedLinear(nn.Module):
             if n > 512:
                 ws = _absmax_workspace(x_work, n, k)
                 d.workspace, d.workspace_elems = ws.data_ptr(), ws.numel()
-            if memo is not None:
-                memo.put(x, share, id(self), codes)
         out = torch.empty((n, self.M_orig), device=dev, dtype=out_dtype)
         d.x, d.out, d.stream = x_work.data_ptr(), out.data_ptr(), stream
         d.x_blocked = codes.data_ptr()
@@ -415,6 +413,8 @@ class MixedLinear(nn.Module):
         rc = nat.lib().tq_prompt_forward(ctypes.byref(d))
         if rc:
             nat.check(rc, "tq_prompt_forward")
+        if d.quantize and memo is not None:   # launched: whoever takes the codes now launches behind them
+            memo.put(x, share, id(self), codes)
         return out
 
     def token_blocked_codes(self, n_rows: int) -> bool:
