@@ -113,3 +113,18 @@ def test_codes_are_not_shared_before_their_launch(library):
         library.before = other_thread
         assert _call(a, x) == 5
     assert seen == [5] and library.quantized == [True, True]
+
+
+@pytest.mark.parametrize("inside", [True, False])
+def test_an_input_changed_in_place_is_quantized_again(library, inside):
+    """Tensors made under inference mode have no version counter: an in-place
+    change between two siblings cannot be seen, so their codes are not shared."""
+    a, b = _siblings()
+    with torch.inference_mode(inside):
+        x = _input(2)
+    with torch.inference_mode():
+        assert x.is_inference() == inside
+        assert _call(a, x) == 2
+        x.mul_(2)
+        assert _call(b, x) == 4
+    assert library.quantized == [True, True]

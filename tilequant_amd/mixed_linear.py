@@ -97,8 +97,8 @@ _LINEAR_FORWARD = [None]
 
 def _view_key(t: torch.Tensor) -> Tuple[Any, ...]:
     """What makes two uses of a tensor see the same values: its storage view
-    and its version counter (inference tensors have none; they cannot be
-    modified in place outside inference mode either)."""
+    and its version counter.  Inference tensors have none, so this does not
+    tell whether one was changed in place (``_shareable``)."""
     version = None if t.is_inference() else int(t._version)
     return (t.data_ptr(), t.storage_offset(), tuple(t.shape), tuple(t.stride()), t.dtype, t.device, version)
 
@@ -168,6 +168,13 @@ def _shared_quant(index: int, stream: int) -> ServeOnce:
     return memo
 
 
+def _shareable(x: torch.Tensor) -> bool:
+    """Whether sibling projections may share ``x``'s codes: under inference
+    mode, for inputs whose version counter tells when they are changed in
+    place (tensors made under inference mode have none)."""
+    return torch.is_inference_mode_enabled() and not x.is_inference()
+
+
 def _blockable(x_work: torch.Tensor) -> bool:
     """Rows the token-blocked quantizer takes: full 64-column tiles, unit
     column stride, 16-byte aligned rows."""
@@ -184,11 +191,9 @@ def _quantize(x_work: torch.Tensor, tile_n: int, blocked: bool) -> Tuple[torch.T
 def _quantize_for(module: nn.Module, x: torch.Tensor, x_work: torch.Tensor,
                   blocked: bool = False) -> Tuple[torch.Tensor, torch.Tensor]:
     """Codes and scales of ``x_work`` (the 2-D view of ``x``) for ``module``
-    (token-blocked when ``blocked``), shared with its sibling projections
-    under inference mode for inputs of at least ACTIVATION_QUANT_CACHE_MIN_ROWS
-    rows."""
-    if x_work.shape[0] < ACTIVATION_QUANT_CACHE_MIN_ROWS or not x_work.is_cuda \
-            or not torch.is_inference_mode_enabled():
+    (token-blocked when ``blocked``), shared with its sibling projections for
+    ``_shareable`` inputs of at least ACTIVATION_QUANT_CACHE_MIN_ROWS rows."""
+    if x_work.shape[0] < ACTIVATION_QUANT_CACHE_MIN_ROWS or not x_work.is_cuda or not _shareable(x):
         return _quantize(x_work, module.tile_n, blocked)
     memo = _shared_quant(x_work.device.index or 0, torch.cuda.current_stream(x_work.device).cuda_stream)
     key = (_view_key(x), module.tile_n, blocked)
@@ -369,8 +374,8 @@ class MixedLinear(nn.Module):
 
     def _prompt_forward(self, x: torch.Tensor, x_work: torch.Tensor) -> torch.Tensor:
         """Prompt-size forward on token-blocked codes: one foreign call that
-        quantizes (unless a sibling projection already has, under inference
-        mode) and multiplies, from a descriptor validated once per shape and
+        quantizes (unless a sibling projection already has, ``_shareable``)
+        and multiplies, from a descriptor validated once per shape and
         set of weight tensors (four calls of a layer at 128 rows took 219 us on
         the host otherwise, for 85 us of kernels)."""
         n, k = x_work.shape
@@ -392,7 +397,7 @@ class MixedLinear(nn.Module):
             launch = self._prompts[key] = self._build_prompt(x_work, out_dtype, order)
         codes_bytes = token_blocked_elems(n, k)
         codes = memo = None
-        if torch.is_inference_mode_enabled():
+        if _shareable(x):
             memo = _shared_quant(index, stream)
             share = (_view_key(x), self.tile_n, "prompt")
             codes = memo.take(x, share, id(self))
@@ -583,7 +588,12 @@ class MixedLinearGroup(nn.Module):
     rows (``concat_packs_along_rows``), one quantization and one GEMM per
     activation, each member served its column slice of the stacked output.
     Every output element comes from the same tile sequence and arithmetic as
-    the member's own MixedLinear, so slices equal the members bitwise."""
+    the member's own MixedLinear, so slices equal the members bitwise.
+
+    The members of one pass are called on one unchanged activation.  A change
+    in place between two members is seen by the version counter; a tensor made
+    under inference mode has none, so there it is the caller's to call the
+    group afresh (``reset_pending``)."""
 
     def __init__(self, members):
         super().__init__()
