@@ -63,6 +63,12 @@ const char* tq_error_string(int code);
 /* ABI version of this header (bumped on any signature change). */
 int tq_abi_version(void);
 
+/* Which graph capture `stream` is in: 0 when none, the capture's id (unique in
+ * the process, shared by the streams that joined it) while it is active, -1
+ * when that cannot be told (an invalidated capture, or the null stream during
+ * another stream's).  Enqueues nothing. */
+int64_t tq_stream_capture_id(void* stream);
+
 /* ---- activation quantization ------------------------------------------
  * Per 64-column tile c of x [n, k]:  a = max |x[:, 64c:64c+64]| over ALL n
  * rows;  sx[c] = 1 if a == 0 else f32(round_to_x_dtype(f32(a) / 127));

@@ -38,6 +38,10 @@ class _Library:
         return 0
 
     @staticmethod
+    def tq_stream_capture_id(stream):
+        return 0
+
+    @staticmethod
     def tq_error_string(code):
         return b"forced by the test"
 
@@ -128,3 +132,39 @@ def test_an_input_changed_in_place_is_quantized_again(library, inside):
         x.mul_(2)
         assert _call(b, x) == 4
     assert library.quantized == [True, True]
+
+
+def test_codes_do_not_cross_a_graph_capture(library, monkeypatch):
+    """Codes of an eager call are not taken inside a capture (its graph would
+    hold no quantization), nor those of a capture outside it or in another
+    one (its launches are only recorded); siblings of one capture share."""
+    now = [0]
+    monkeypatch.setattr(ml.nat, "capture_id", lambda stream: now[0])
+    a, b = _siblings()
+    with torch.inference_mode():
+        for first, second in ((0, 7), (7, 0), (7, 9), (7, 7), (None, None)):
+            with torch.inference_mode(False):
+                x = _input(2)
+            library.quantized.clear()
+            now[0] = first
+            _call(a, x)
+            now[0] = second
+            _call(b, x)
+            assert library.quantized == [True, first != second or first is None], (first, second)
+
+
+def test_group_outputs_do_not_cross_a_graph_capture(library, monkeypatch):
+    now, calls = [0], []
+    monkeypatch.setattr(ml.nat, "capture_id", lambda stream: now[0])
+    group = ml.MixedLinearGroup(_siblings())
+    group.linear.forward = lambda x: calls.append(now[0]) or torch.zeros(ROWS, 256)
+    x = _input(2)
+    for first, second, want in ((0, 0, [0]), (0, 7, [0, 7]), (7, 0, [7, 0]), (7, 9, [7, 9]), (7, 7, [7]),
+                                (None, None, [None, None])):
+        calls.clear()
+        group.reset_pending()
+        now[0] = first
+        group.output_for(x, 0)
+        now[0] = second
+        group.output_for(x, 1)
+        assert calls == want

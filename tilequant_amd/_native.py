@@ -36,6 +36,7 @@ _SIGNATURES = {
     "tq_act_quant_token_blocked": (_i, [_p, _i64, _i, _i, _i, _p, _p, _p]),
     "tq_gemm_prefers_token_blocked": (_i, [_i, _i, _i, _i]),
     "tq_read_probe": (_i, [_p, _i64, _p, _p]),
+    "tq_stream_capture_id": (_i64, [_p]),
     "tq_act_quant_blocked": (_i, [_p, _i64, _i, _i, _i, _p, _p, _p, _i64, _p]),
     "tq_gemm_mixed_blocked": (_i, [_p, _p,
                                    _p, _p, _p, _p,
@@ -218,6 +219,13 @@ def require_device(*tensors: torch.Tensor) -> None:
 
 def stream_handle(device: torch.device) -> int:
     return int(torch.cuda.current_stream(device).cuda_stream)
+
+
+def capture_id(stream: int) -> Optional[int]:
+    """The graph capture that ``stream`` is in: 0 for none, its id, or None when
+    that cannot be told."""
+    found = int(lib().tq_stream_capture_id(stream))
+    return None if found < 0 else found
 
 
 def ptr(t: Optional[torch.Tensor]) -> Optional[int]:

@@ -3,6 +3,17 @@
 
 extern "C" int tq_abi_version(void) { return 3; }
 
+extern "C" int64_t tq_stream_capture_id(void* stream) {
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  unsigned long long id = 0;
+  if (hipStreamGetCaptureInfo(static_cast<hipStream_t>(stream), &status, &id) != hipSuccess) {
+    (void)hipGetLastError();   // not a launch's error: the next launch must not report it
+    return -1;
+  }
+  if (status == hipStreamCaptureStatusNone) return 0;
+  return status == hipStreamCaptureStatusActive && id != 0 ? (int64_t)id : -1;
+}
+
 extern "C" const char* tq_error_string(int code) {
   switch (code) {
     case TQ_OK: return "ok";

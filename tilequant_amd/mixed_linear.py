@@ -175,6 +175,15 @@ def _shareable(x: torch.Tensor) -> bool:
     return torch.is_inference_mode_enabled() and not x.is_inference()
 
 
+def _share_key(x: torch.Tensor, stream: int, *what) -> Optional[Tuple[Any, ...]]:
+    """Key of something computed from ``x`` on ``stream``: its view and the graph
+    capture the stream is in, if any.  A capture's launches run when its graph
+    is replayed, so what it computes serves its own later calls only, and what
+    eager calls computed does not serve it.  None: not to be shared."""
+    capture = nat.capture_id(stream)
+    return None if capture is None else (_view_key(x), capture) + what
+
+
 def _blockable(x_work: torch.Tensor) -> bool:
     """Rows the token-blocked quantizer takes: full 64-column tiles, unit
     column stride, 16-byte aligned rows."""
@@ -195,13 +204,15 @@ def _quantize_for(module: nn.Module, x: torch.Tensor, x_work: torch.Tensor,
     ``_shareable`` inputs of at least ACTIVATION_QUANT_CACHE_MIN_ROWS rows."""
     if x_work.shape[0] < ACTIVATION_QUANT_CACHE_MIN_ROWS or not x_work.is_cuda or not _shareable(x):
         return _quantize(x_work, module.tile_n, blocked)
-    memo = _shared_quant(x_work.device.index or 0, torch.cuda.current_stream(x_work.device).cuda_stream)
-    key = (_view_key(x), module.tile_n, blocked)
-    hit = memo.take(x, key, id(module))
+    stream = torch.cuda.current_stream(x_work.device).cuda_stream
+    memo = _shared_quant(x_work.device.index or 0, stream)
+    key = _share_key(x, stream, module.tile_n, blocked)
+    hit = memo.take(x, key, id(module)) if key is not None else None
     if hit is not None:
         return hit
     codes = _quantize(x_work, module.tile_n, blocked)
-    memo.put(x, key, id(module), codes)
+    if key is not None:
+        memo.put(x, key, id(module), codes)
     return codes
 
 
@@ -396,10 +407,10 @@ class MixedLinear(nn.Module):
                 self._prompts.pop(next(iter(self._prompts)), None)
             launch = self._prompts[key] = self._build_prompt(x_work, out_dtype, order)
         codes_bytes = token_blocked_elems(n, k)
-        codes = memo = None
-        if _shareable(x):
+        codes = None
+        share = _share_key(x, stream, self.tile_n, "prompt") if _shareable(x) else None
+        if share is not None:
             memo = _shared_quant(index, stream)
-            share = (_view_key(x), self.tile_n, "prompt")
             codes = memo.take(x, share, id(self))
         # a copy per call: concurrent callers never patch one descriptor
         d = nat.PromptDesc.from_buffer_copy(launch.desc)
@@ -418,7 +429,7 @@ class MixedLinear(nn.Module):
         rc = nat.lib().tq_prompt_forward(ctypes.byref(d))
         if rc:
             nat.check(rc, "tq_prompt_forward")
-        if d.quantize and memo is not None:   # launched: whoever takes the codes now launches behind them
+        if d.quantize and share is not None:   # launched: whoever takes the codes now launches behind them
             memo.put(x, share, id(self), codes)
         return out
 
@@ -611,11 +622,12 @@ class MixedLinearGroup(nn.Module):
     def output_for(self, x: torch.Tensor, index: int) -> torch.Tensor:
         """Stacked output for ``x``: computed when member ``index`` is the
         first to ask for this activation (or asks again), reused otherwise."""
-        key = _view_key(x)
-        out = self._shared.take(x, key, index)
+        key = _share_key(x, torch._C._cuda_getCurrentRawStream(x.device.index) if x.is_cuda else 0)
+        out = self._shared.take(x, key, index) if key is not None else None
         if out is None:
             out = self.linear(x)
-            self._shared.put(x, key, index, out)
+            if key is not None:
+                self._shared.put(x, key, index, out)
         return out
 
     def reset_pending(self) -> None:
