@@ -168,3 +168,37 @@ def test_group_outputs_do_not_cross_a_graph_capture(library, monkeypatch):
         now[0] = second
         group.output_for(x, 1)
         assert calls == want
+
+
+def test_a_lookup_never_returns_another_inputs_value():
+    """Threads on one stream share a memo: another thread's put between a
+    lookup's checks and its result must not reach the lookup's caller."""
+    memo, x, other = ml.ServeOnce(), torch.zeros(2), torch.ones(2)
+
+    class Key:
+        def __eq__(self, rhs):
+            memo.put(other, "key of the other", "a", "codes of the other")
+            return True
+
+        def __ne__(self, rhs):
+            return not self == rhs
+
+    memo.put(x, Key(), "a", "codes of x")
+    assert memo.take(x, "key", "b") in (None, "codes of x")
+    memo.put(x, "key", "a", "codes of x")
+    assert memo.take(x, "key", "b") == "codes of x"
+
+
+def test_a_memo_copies_empty():
+    import copy
+    import pickle
+
+    memo, x = ml.ServeOnce(consumers=3), torch.zeros(2)
+    memo.put(x, "key", "a", "codes of x")
+    for other in (copy.deepcopy(memo), pickle.loads(pickle.dumps(memo))):
+        assert other.consumers == 3 and other.take(x, "key", "b") is None
+    # as modules saved by earlier versions hold it: one state entry per field
+    old = ml.ServeOnce.__new__(ml.ServeOnce)
+    old.__setstate__((None, {"consumers": 2, "_source": None, "_key": None, "_taken": frozenset(), "_value": None}))
+    assert old.consumers == 2 and old.take(x, "key", "b") is None
+    assert memo.take(x, "key", "b") == "codes of x"

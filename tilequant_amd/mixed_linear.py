@@ -119,25 +119,37 @@ class ServeOnce:
     mixed_linear.py:24-111), and the stacked output of a projection group
     shared by its members (mixed_linear.py:257-333)."""
 
-    __slots__ = ("consumers", "_source", "_key", "_taken", "_value")
+    # (source reference, key, consumers served, value) or None: one object, read
+    # and replaced whole, so threads sharing a memo never see halves of two.
+    __slots__ = ("consumers", "_entry")
 
     def __init__(self, consumers: Optional[int] = None) -> None:
         self.consumers = consumers
-        self.clear()
+        self._entry = None
+
+    # a copy starts empty: the value belongs to this memo's tensors
+    def __getstate__(self):
+        return None, {"consumers": self.consumers}
+
+    def __setstate__(self, state):
+        self.__init__(state[1]["consumers"])
 
     def clear(self) -> None:
-        self._source = None
-        self._key = None
-        self._taken: frozenset = frozenset()
-        self._value = None
+        self._entry = None
+
+    @property
+    def _value(self):
+        entry = self._entry
+        return None if entry is None else entry[3]
 
     def take(self, source: torch.Tensor, key, consumer) -> Optional[Any]:
-        if self._source is None or self._source() is not source or self._key != key or consumer in self._taken:
+        entry = self._entry
+        if entry is None or entry[0]() is not source or entry[1] != key or consumer in entry[2]:
             return None
-        value = self._value
-        self._taken = self._taken | {consumer}
-        if self.consumers is not None and len(self._taken) >= self.consumers:
-            self.clear()
+        ref, kept, served, value = entry
+        served = served | {consumer}
+        done = self.consumers is not None and len(served) >= self.consumers
+        self._entry = None if done else (ref, kept, served, value)
         return value
 
     def put(self, source: torch.Tensor, key, consumer, value) -> None:
@@ -146,14 +158,15 @@ class ServeOnce:
             return
 
         def released(ref, memo=self):
-            if memo._source is ref:
-                memo.clear()
+            entry = memo._entry
+            if entry is not None and entry[0] is ref:
+                memo._entry = None
 
         try:
-            self._source = weakref.ref(source, released)
+            ref = weakref.ref(source, released)
         except TypeError:
             return
-        self._key, self._taken, self._value = key, frozenset((consumer,)), value
+        self._entry = (ref, key, frozenset((consumer,)), value)
 
 
 # One memo per (device, stream): kernels on one stream run in order, so codes
