@@ -6,9 +6,11 @@ import re
 import struct
 import subprocess
 from pathlib import Path
+from types import SimpleNamespace
 
 import numpy as np
 import pytest
+import torch
 
 from tilequant_amd import _native as nat
 
@@ -127,3 +129,29 @@ def test_ring_slices_land_before_the_first_barrier_publishes_them(tmp_path):
                     i = index[ins[i - 1][0] + 4 + 4 * ((int(jump[1], 0) + 0x8000) % 0x10000 - 0x8000)]
             assert landed, f"{name}: the first ring barrier is passed with {since} later operations and no wait"
         assert bodies >= 3, name         # 1, 2 or 4 token blocks, and the 16-bit-heavy row tiles
+
+
+def test_modules_saved_whole_before_prompt_descriptors_still_load():
+    """A module object pickled by a version without prompt descriptors and slot
+    orders lacks both in its state."""
+    import pickle
+
+    from test_host_logic import _cpu_pack
+
+    from tilequant_amd.gemm_rows_splitk_64x64 import PrefillPlan
+    from tilequant_amd.mixed_linear import MixedLinear
+
+    lin = MixedLinear(_cpu_pack(128, 192, 0.3, 1)[0], None, SimpleNamespace(dtype_out="bf16"))
+    state = dict(lin.__dict__, _launches={})
+    del state["_prompts"]
+    old = MixedLinear.__new__(MixedLinear)
+    old.__setstate__(state)
+    assert old._prompts == {} and torch.equal(old.int8_tiles, lin.int8_tiles)
+    again = pickle.loads(pickle.dumps(old))
+    assert again._prompts == {} and again._launches == {}
+    units = torch.arange(3, dtype=torch.int32)
+    plan = PrefillPlan.__new__(PrefillPlan)
+    plan.__setstate__((None, {"units": units, "n_first": 1, "n_tr": 3}))
+    assert plan.units is units and (plan.n_first, plan.n_tr, plan.row_order) == (1, 3, None)
+    plan = pickle.loads(pickle.dumps(PrefillPlan(units, 2, 3, row_order=units)))
+    assert (plan.n_first, plan.row_order.tolist()) == (2, [0, 1, 2])

@@ -92,6 +92,10 @@ class PrefillPlan:
         self.units, self.n_first, self.n_tr = units, int(n_first), int(n_tr)
         self.row_order = row_order   # slots of the blocked GEMM (tq_gemm_row_order; None: row tiles in order)
 
+    def __setstate__(self, state):   # plans pickled by earlier versions have no row_order
+        fields = state[1]
+        self.__init__(fields["units"], fields["n_first"], fields["n_tr"], fields.get("row_order"))
+
 
 def prefill_plan(*, int8_tile_ids: torch.Tensor, int8_row_ptr: torch.Tensor, fp16_row_ptr: torch.Tensor,
                  n_tr: int, n_tc: int, device=None) -> Optional[PrefillPlan]:

@@ -291,6 +291,10 @@ class MixedLinear(nn.Module):
         # a copy starts without descriptors: they hold this module's addresses
         return dict(self.__dict__, _launches={}, _prompts={})
 
+    def __setstate__(self, state):
+        # modules saved whole by earlier versions lack what came later
+        super().__setstate__({"_launches": {}, "_prompts": {}, "_blocked_rows": {}, "_plan": None, **state})
+
     # the tile storage order travels with the state_dict
     def get_extra_state(self):
         return {"tile_layout": self.tile_layout}
