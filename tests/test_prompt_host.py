@@ -155,3 +155,19 @@ def test_modules_saved_whole_before_prompt_descriptors_still_load():
     assert plan.units is units and (plan.n_first, plan.n_tr, plan.row_order) == (1, 3, None)
     plan = pickle.loads(pickle.dumps(PrefillPlan(units, 2, 3, row_order=units)))
     assert (plan.n_first, plan.row_order.tolist()) == (2, [0, 1, 2])
+
+
+@pytest.mark.parametrize("heavy,n16,rest", [([5], 33, 2), (list(range(28)), 48, 0), (list(range(0, 48, 2)), 48, 0)])
+def test_plans_order_heavy_row_tiles_that_split_no_pair(heavy, n16, rest):
+    """Row tiles mostly in 16 bits get slots of their own also where the pair
+    plan of the row-major kernel splits nothing (48 x 48 tiles: one row tile
+    with 33 in 16 bits among others with 2, the first 28 all in 16 bits, every
+    second one)."""
+    from test_host_logic import _plan_from_ids16
+
+    plan = _plan_from_ids16(np.concatenate([r * 48 + np.arange(n16 if r in heavy else rest) for r in range(48)]), 48, 48)
+    assert plan.units is None and plan.n_tr == 48
+    slots = plan.row_order.tolist()
+    whole = -(-len(heavy) // 4) * 4
+    assert slots[:whole] == heavy + [-1] * (whole - len(heavy))
+    assert slots[whole:] == [r for r in range(48) if r not in heavy]

@@ -78,17 +78,18 @@ def _fused_workspace(device, n, M, K, n_tr, n_tc, split_k):
 
 
 class PrefillPlan:
-    """Work plan for the prefill GEMM over one packed weight: ``units`` (a
-    device int32 tensor) lists row-tile pairs and single row tiles (value
-    row | 1 << 30), in dispatch order; the first ``n_first`` units take all
-    their token blocks before the others start; ``n_tr`` is the row-tile
-    count of the weight it covers (every row tile exactly once).
+    """Work plan for the prefill GEMMs over one packed weight: ``units`` (a
+    device int32 tensor, or None: the row-tile pairs in order) lists row-tile
+    pairs and single row tiles (value row | 1 << 30), in dispatch order; the
+    first ``n_first`` units take all their token blocks before the others
+    start; ``n_tr`` is the row-tile count of the weight it covers (every row
+    tile exactly once).
     ``prefill_plan`` builds one from the row pointers; the outputs do not
     depend on it, as long as it covers the weight's row tiles."""
 
     __slots__ = ("units", "n_first", "n_tr", "row_order")
 
-    def __init__(self, units: torch.Tensor, n_first: int, n_tr: int, row_order: Optional[torch.Tensor] = None):
+    def __init__(self, units: Optional[torch.Tensor], n_first: int, n_tr: int, row_order: Optional[torch.Tensor] = None):
         self.units, self.n_first, self.n_tr = units, int(n_first), int(n_tr)
         self.row_order = row_order   # slots of the blocked GEMM (tq_gemm_row_order; None: row tiles in order)
 
@@ -101,8 +102,10 @@ def prefill_plan(*, int8_tile_ids: torch.Tensor, int8_row_ptr: torch.Tensor, fp1
                  n_tr: int, n_tc: int, device=None) -> Optional[PrefillPlan]:
     """Plan the prefill GEMM's work units from the pack's tile bookkeeping:
     row-tile pairs whose many 16-bit tiles would make them finish long after
-    the others are split into single row tiles (row order kept).  Returns
-    None when no pair needs splitting.
+    the others are split into single row tiles (row order kept).  The plan's
+    ``row_order`` gives the token-blocked GEMM's row tiles that are mostly in 16
+    bits workgroups of their own.  Returns None when no pair needs splitting
+    and no row tile is mostly in 16 bits.
     Copies the row pointers and INT8 ids to the host (a synchronisation):
     call it once per weight, outside graph capture."""
     n_tr, n_tc = int(n_tr), int(n_tc)
@@ -119,15 +122,15 @@ def prefill_plan(*, int8_tile_ids: torch.Tensor, int8_row_ptr: torch.Tensor, fp1
         ctypes.byref(n_first))
     if rc < 0:   # a count otherwise
         nat.check(rc, "tq_gemm_prefill_plan")
-    if rc == 0:
-        return None
     slots = 0
-    if rp16 is not None:
+    if rp16 is not None and (rc > 0 or bool((3 * rp16[:n_tr + 1].diff() >= 2 * n_tc).any())):
         slots = nat.lib().tq_gemm_row_order(rp16.data_ptr(), n_tr, n_tc, units[rc:].data_ptr(), n_tr + 3)
         if slots < 0:
             nat.check(slots, "tq_gemm_row_order")
+    if rc + slots == 0:
+        return None
     both = units[:rc + slots].to(device if device is not None else int8_row_ptr.device)
-    return PrefillPlan(both[:rc], n_first.value, n_tr, both[rc:] if slots else None)
+    return PrefillPlan(both[:rc] if rc else None, n_first.value, n_tr, both[rc:] if slots else None)
 
 
 def _check_tiles(name: str, t: torch.Tensor, dtype) -> None:
@@ -227,10 +230,11 @@ def gemm_mixed_rows_splitk(
     units = None
     if prefill_plan is not None:
         units = prefill_plan.units
-        if units.device != x_fp.device or units.dtype != torch.int32 or not units.is_contiguous():
+        if units is not None and (units.device != x_fp.device or units.dtype != torch.int32
+                                  or not units.is_contiguous()):
             raise ValueError("prefill_plan.units must be a contiguous int32 tensor on the input's device")
-        if (prefill_plan.n_tr != n_tr or not 0 < units.numel() <= n_tr
-                or not 0 <= prefill_plan.n_first <= units.numel()):
+        if prefill_plan.n_tr != n_tr or units is not None and (
+                not 0 < units.numel() <= n_tr or not 0 <= prefill_plan.n_first <= units.numel()):
             raise ValueError(f"prefill_plan covers {prefill_plan.n_tr} row tiles, the weight has {n_tr}")
     if _products is not None:   # test-only DUMP launch (gemm_mixed_rows_products_i32)
         prod, row0, rows, kernel = _products
