@@ -212,9 +212,11 @@ int tq_gemm_prefill_plan(const int32_t* int8_row_ptr, const int32_t* int8_tile_i
 
 /* The GEMM for prompt sizes on token-blocked codes of any number of rows
  * (tq_act_quant_blocked): x_blocked, 16 ceil(n / 16) * k bytes.  k = 64 * n_tc,
- * n_tc <= 304, 16-byte aligned x_fp rows (x_fp_stride_n % 8 == 0).  The outputs
- * are bitwise those of tq_gemm_mixed_rows on the same codes row-major for
- * n > 64.  row_order (nullable, device, n_slots entries): the row tiles 0 ..
+ * n_tc <= 304, 16-byte aligned x_fp rows (x_fp_stride_n % 8 == 0).  For more
+ * than 384 tokens (more than 1280 from 96 column tiles on) the outputs are
+ * bitwise those of tq_gemm_mixed_rows on the same codes row-major; up to there
+ * a row tile's tiles are summed in 4 or 8 fp32 partial sums, added in a fixed
+ * order, so outputs differ from those by fp32 rounding.  row_order (nullable, device, n_slots entries): the row tiles 0 ..
  * n_tr - 1, each once, and -1 for empty slots; consecutive groups of four
  * slots share a workgroup, so row tiles with alike 16-bit tile counts are best
  * neighbours (any such list gives the same outputs).  products / row0 /

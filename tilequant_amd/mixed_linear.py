@@ -12,8 +12,13 @@ projection groups and sibling-activation cache as the reference
   reference's is 4096): the INT8 copy of even a 16384 x 18944 input is 310 MB,
   small against 288 GB of HBM, and one GEMM launch over a whole 8192-token
   prefill fills the GPU better than two (measured 16% faster per layer).
-  Chunking never changes the output: the scales are over the whole input
-  either way and rows are independent.
+  Chunking never changes scales or codes: the scales are over the whole
+  input either way and rows are independent.  Which fp32 partial sums an
+  output is added from depends on the rows of a launch (above 384 rows, 1280
+  for inputs of 96 column tiles or more, one sum in the reference's order;
+  up to there 4 or 8, for whole aligned inputs of more than 64 rows), so a
+  chunked input of such a size, or one with a last chunk of at most 64 rows,
+  differs from the unchunked one by fp32 rounding.
 * Q/K/V and Gate/Up siblings can be stacked into one ``MixedLinearGroup``
   (one quantization + one GEMM per group), each member served a column slice.
 
