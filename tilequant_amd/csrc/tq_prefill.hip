@@ -1,10 +1,13 @@
 // tq_prefill.hip -- mixed INT8/16-bit tile GEMM for more than 64 tokens on
 // token-blocked activation codes (tq_gemm_mixed_blocked).
 //
-// Same sums as the row-major prefill kernels of tq_gemm.hip, bit for bit: one
-// fp32 accumulator per output, the INT8 tiles of a row tile by column (exact
-// INT32 tile product, then one FMA by sx[c] * sw[t]), then its 16-bit tiles by
-// position (the reference's loop, gemm_rows_splitk_64x64.py:125-153).
+// The whole-list kernel forms the sums of the row-major prefill kernels of
+// tq_gemm.hip, bit for bit: one fp32 accumulator per output, the INT8 tiles of
+// a row tile by column (exact INT32 tile product, then one FMA by
+// sx[c] * sw[t]), then its 16-bit tiles by position (the reference's loop,
+// gemm_rows_splitk_64x64.py:125-153).  The split kernel (few tokens, see
+// split_waves) deals a row tile's tiles to 4 or 8 waves and adds their partial
+// sums in wave order, as the decode kernels do.
 #include <algorithm>
 #include <vector>
 
@@ -816,10 +819,14 @@ using namespace tq;
 //     O                  33 -> 10   32 -> 13   33 -> 16   33 -> 18
 //     Gate/Up            38 -> 24   38 -> 33   48 -> 51   50 -> 63
 //   Qwen2.5-7B Gate/Up   56 -> 54   90 -> 70   96 -> 125  142 -> 179
-// so the layer's three together gain up to about 400 tokens.  Long lists (Down)
-// longer, 192 / 1024 / 1500 tokens: Llama 80 -> 26, 77 -> 54, 103 -> 87;
+// Gate/Up alone stops gaining at 200-300 tokens; a layer's three together gain up
+// to the limit, 192 / 320 / 384 tokens with uniform keep05 masks: Llama 103 -> 63,
+// 113 -> 80, 114 -> 91; Qwen2.5-7B 149 -> 104, 171 -> 153, 177 -> 166; 14B 183 -> 126,
+// 206 -> 178, 232 -> 204; with clustered keep10 masks at 384 7B loses (183 -> 191),
+// 14B gains (236 -> 223).  The row-major kernels take 198-371 there.  Long lists
+// (Down) longer, 192 / 1024 / 1500 tokens: Llama 80 -> 26, 77 -> 54, 103 -> 87;
 // Qwen2.5-7B 174 -> 51, 173 -> 139, 229 -> 219; 14B 131 -> 41, 173 -> 131, 183 ->
-// 221.  Eight waves where the list is long and the grid small (192 tokens: 24,
+// 221; at the limit of 1280 78, 194, 197 against 82, 236, 182.  Eight waves where the list is long and the grid small (192 tokens: 24,
 // 46 and 39 against 26, 51 and 41 us; at 384 39, 84, 67 against 34, 76, 63).
 constexpr int kSplitTokens = 384, kSplitLongTokens = 1280, kSplitLongTiles = 96, kSplitWideTokens = 256;
 static int split_waves(int n, int n_tc) {
@@ -836,7 +843,10 @@ static int split_waves(int n, int n_tc) {
 // on, 128 tokens wherever a CU gets two of them: 64-token workgroups read the
 // weights twice as often, and those of so many units do not stay in the L2s
 // (Qwen2.5-7B Gate/Up at 777 / 2048 / 8192 tokens 268 / 669 / 2697 vs 229 / 476 /
-// 1869 us).
+// 1869 us).  Lists of other lengths scale both sides: over the four projections
+// of Llama-3.2-3B, Qwen2.5-7B and 14B (48 to 296 tiles) at 400 to 4096 tokens the
+// rule takes the faster side at 84 of 87 points and loses 1, 5 and 16% (Llama
+// Gate/Up at 600 tokens, 81 vs 70 us) at the others.
 static int blocked_tb(int n, int units) {
   constexpr int kCus = 256, kManyUnits = 64;
   const int64_t l2 = ((int64_t)units * ((n + 63) / 64) + kCus - 1) / kCus;
