@@ -202,3 +202,27 @@ def test_a_memo_copies_empty():
     old.__setstate__((None, {"consumers": 2, "_source": None, "_key": None, "_taken": frozenset(), "_value": None}))
     assert old.consumers == 2 and old.take(x, "key", "b") is None
     assert memo.take(x, "key", "b") == "codes of x"
+
+
+def test_an_outgrown_absmax_workspace_stays_alive(monkeypatch):
+    """A captured graph holds the partial-max workspace by address: a larger
+    input replaces the buffer, the old one is kept."""
+    import gc
+    import weakref
+
+    from tilequant_amd import quantize_activation as qa
+
+    need = [100]
+    monkeypatch.setattr(qa.nat, "lib", lambda: SimpleNamespace(tq_act_absmax_workspace_elems=lambda n, k: need[0]))
+    monkeypatch.setattr(qa.nat, "stream_handle", lambda device: 0)
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
+    monkeypatch.setattr(qa, "_WORKSPACE", {})
+    monkeypatch.setattr(qa, "_RETIRED", [], raising=False)
+    x = torch.zeros(2, 64)
+    first = qa._absmax_workspace(x, 600, 64)
+    assert qa._absmax_workspace(x, 600, 64) is first
+    need[0], alive = first.numel() + 1, weakref.ref(first)
+    del first
+    assert qa._absmax_workspace(x, 20000, 64).numel() >= need[0]
+    gc.collect()
+    assert alive() is not None

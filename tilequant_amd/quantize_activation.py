@@ -7,13 +7,14 @@ taken over ALL rows of the call.
 """
 from __future__ import annotations
 
-from typing import Dict, Tuple
+from typing import Dict, List, Tuple
 
 import torch
 
 from . import _native as nat
 
 _WORKSPACE: Dict[Tuple[int, int], torch.Tensor] = {}
+_RETIRED: List[torch.Tensor] = []   # outgrown workspaces: a captured graph may hold their addresses
 
 
 def _absmax_workspace(x: torch.Tensor, n: int, k: int) -> torch.Tensor:
@@ -24,7 +25,11 @@ def _absmax_workspace(x: torch.Tensor, n: int, k: int) -> torch.Tensor:
     key = (dev.index if dev.index is not None else torch.cuda.current_device(), nat.stream_handle(dev))
     ws = _WORKSPACE.get(key)
     if ws is None or ws.numel() < need:
-        ws = torch.empty((max(need, 1 << 14),), device=dev, dtype=torch.float32)
+        size = max(need, 1 << 14)
+        if ws is not None:
+            _RETIRED.append(ws)
+            size = max(size, 2 * ws.numel())   # so that the retired ones together stay below the current one
+        ws = torch.empty((size,), device=dev, dtype=torch.float32)
         _WORKSPACE[key] = ws
     return ws
 
